@@ -167,6 +167,19 @@ struct hfh_tsweep {
     int kmax = 0;              // most entries of any lane
 };
 
+// SGS / ILU0 on a 5- / 7-point natural-order grid: the sweeps by pencils of
+// 64 lines along x (hfh_pencil.hip).
+struct hfh_pencil {
+    int np = 0;                // pencils (0: none)
+    int nx = 0, ny = 0, nz = 0, npy = 0, npz = 0;
+    int ng = 0;                // groups of 4 steps of a pencil
+    int *order = nullptr;      // device: pencils in dependency order
+    void *fval = nullptr, *bval = nullptr;   // forward / backward values by (pencil, step, lane)
+    void *y = nullptr;         // forward results by (pencil, step, lane)
+    void *fbox = nullptr, *bbox = nullptr;   // face values received by each pencil
+    int *ctl = nullptr;        // tickets, slow-division flag
+};
+
 struct hfh_prec {
     int kind = HFH_PREC_NONE;
     hfh_ctx *ctx = nullptr;
@@ -183,6 +196,7 @@ struct hfh_prec {
     hfh_sweep fw, bw;               // MC-SGS: lower-colour / upper-colour entries per row
     hfh_tsweep tlo, tup;            // SGS / ILU0: forward / backward sweep rows by level
     hfh_tsweep blo, bup;            // SGS / ILU0 on a structured grid: the sweeps by geometric block
+    hfh_pencil pen;                 // SGS / ILU0 on a 5- / 7-point grid: by pencils instead of blocks
     unsigned tversion = 0;          // A->version the sweep values were copied at
     // SGS / ILU0 outside the fused drivers: both sweeps captured once as a
     // hipGraph on internal in/out buffers (one launch instead of one per level)
@@ -279,6 +293,15 @@ int mcsgs_rz_slots(const hfh_prec *P);
 // Brings a preconditioner's copies of the matrix values up to date (after the
 // matrix's values changed); a no-op while the stream is being captured.
 int prec_sync(hfh_prec *P);
+
+// SGS / ILU0 sweeps by pencils (hfh_pencil.hip).  pencil_build leaves P->pen
+// empty where the pattern is not a full 5- / 7-point stencil of the grid
+// (nx, and nxy in 3D, else 0); pencil_fill copies the matrix's values;
+// pencil_apply runs both sweeps (in and out natural order, not aliased).
+int pencil_build(hfh_prec *P, int nx, long long nxy);
+int pencil_fill(hfh_prec *P);
+void pencil_free(hfh_pencil &G);
+int pencil_apply(hfh_prec *P, const void *in, void *out, const int *done);
 
 // XCD-aware workgroup remap: consecutive logical tiles land on one XCD so its
 // L2 keeps the shared gather window.
