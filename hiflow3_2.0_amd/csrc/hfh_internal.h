@@ -105,6 +105,9 @@ struct hfh_csr {
     int sx_chunk = 0;          // elements per chunk (16)
     int sx_img = 0;            // largest image of a slice (chunks * sx_chunk)
     int *diag = nullptr;   // diagonal position per row
+    // longest row and how far its columns reach below / above the row, of
+    // square matrices small enough for the resident CG (else shape_len 0)
+    int shape_len = 0, shape_lo = 0, shape_hi = 0;
     bool has_structure = false;
     bool sorted = true;      // columns ascending in every row (false after a diagonal-first swap)
     unsigned version = 0;    // bumped whenever the values or the structure change
@@ -294,6 +297,15 @@ int mcsgs_rz_slots(const hfh_prec *P);
 // matrix's values changed); a no-op while the stream is being captured.
 int prec_sync(hfh_prec *P);
 
+// CG of a small enough system in one launch (hfh_cgres.hip): x is the initial
+// guess and the result; z0, z1 and slots (n elements each) are work space.
+// *ran false: the system does not qualify and nothing was done.
+constexpr int kResidentRows = 4 * 512 * 256;
+constexpr long long kResidentLds = 158 * 1024;
+template <typename T>
+int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1, void *slots, double *hist,
+                const hfh_control &ctl, hfh_solve_info *info, bool *ran);
+
 // SGS / ILU0 sweeps by pencils (hfh_pencil.hip).  pencil_build leaves P->pen
 // empty where the pattern is not a full 5- / 7-point stencil of the grid
 // (nx, and nxy in 3D, else 0); pencil_fill copies the matrix's values;
@@ -353,6 +365,33 @@ __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
+}
+
+// A 32-bit value moved between lanes by a DPP control (0 where the source
+// lane does not exist or the row is masked out).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0u, static_cast<unsigned>(u), CTRL, ROWS, 0xf, false);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0u, static_cast<unsigned>(u >> 32), CTRL, ROWS, 0xf, false);
+    return __builtin_bit_cast(double, static_cast<unsigned long long>(hi) << 32 | lo);
+}
+
+// Sum over the wave, the same value in every lane: rows of 16 lanes by shifts,
+// then the rows by broadcasts, with vector moves instead of the LDS unit's
+// permutes (a dependent chain of six of those takes about 0.3 us).  Another
+// order of adds than wave_sum.
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+    v += dpp_move<0x111, 0xf>(v);   // row_shr:1
+    v += dpp_move<0x112, 0xf>(v);   // row_shr:2
+    v += dpp_move<0x114, 0xf>(v);   // row_shr:4
+    v += dpp_move<0x118, 0xf>(v);   // row_shr:8
+    v += dpp_move<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+    v += dpp_move<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_readlane(static_cast<unsigned>(u), 63);
+    const unsigned hi = __builtin_amdgcn_readlane(static_cast<unsigned>(u >> 32), 63);
+    return __builtin_bit_cast(double, static_cast<unsigned long long>(hi) << 32 | lo);
 }
 
 __device__ __forceinline__ int wave_max(int v) {

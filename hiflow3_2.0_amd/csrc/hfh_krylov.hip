@@ -1,5 +1,8 @@
 // hfh_krylov.hip -- device-resident Krylov drivers.
 //
+// CG with Jacobi or no preconditioner on a system that fits on the chip runs
+// as one launch (hfh_cgres.hip); the launched form below serves the others.
+//
 // CG (linear_solver/cg.cc:163-248) is restated with its scalars kept in HBM so
 // the host never waits on a Dot.  One Jacobi iteration is three or four launches:
 //   K1  Ap = A p with per-workgroup partial sums of Ap.p (summed by a
@@ -633,6 +636,46 @@ struct PcgWork {
         return HFH_OK;
     }
 
+    // The device residual history into hhist (noalloc: through the context's
+    // 256 pinned result slots, a piece at a time).
+    int fetch_hist(double *hhist, int count, bool noalloc) {
+        hfh_ctx *c = R.A->ctx;
+        if (!noalloc) {
+            HFH_HIP(hipMemcpy(hhist, hist, sizeof(double) * count, hipMemcpyDeviceToHost));
+            return HFH_OK;
+        }
+        for (int k = 0; k < count; k += 256) {
+            const int m = std::min(256, count - k);
+            HFH_HIP(hipMemcpyAsync(c->host_res, hist + k, sizeof(double) * m, hipMemcpyDeviceToHost, c->stream));
+            HFH_HIP(hipStreamSynchronize(c->stream));
+            std::memcpy(hhist + k, c->host_res, sizeof(double) * m);
+        }
+        return HFH_OK;
+    }
+
+    // After a resident solve (the stream has been synchronised).
+    int finish_resident(const hfh_solve_info &ri, hfh_solve_info *info, double *hhist, bool noalloc, hipEvent_t e0,
+                        hipEvent_t e1, std::chrono::steady_clock::time_point t0) {
+        float ms = static_cast<float>(
+            std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count());
+        if (!noalloc) {
+            HFH_HIP(hipEventRecord(e1, R.A->ctx->stream));
+            HFH_HIP(hipEventSynchronize(e1));
+            (void)hipEventElapsedTime(&ms, e0, e1);
+            (void)hipEventDestroy(e0);
+            (void)hipEventDestroy(e1);
+        }
+        have_dir = false;
+        if (hhist) {
+            if (int rc = fetch_hist(hhist, ri.iters + 1, noalloc)) return rc;
+        }
+        if (info) {
+            *info = ri;
+            info->time_ms = ms;
+        }
+        return HFH_OK;
+    }
+
     // Solves A x = b from the given x (device pointers); fills info.
     // x_zero: x holds zeros, so r = b without the SpMV.  keep_direction:
     // continue the previous solve's search direction, p = z + (r.z / r_k.z_k) p
@@ -664,6 +707,14 @@ struct PcgWork {
             HFH_HIP(hipEventRecord(e0, s));
         }
         int rc;
+        // a system that fits on the chip: the whole solve in one launch
+        if (R.mode != 2 && !keep_direction) {
+            hfh_solve_info ri{};
+            bool ran = false;
+            rc = cg_resident<T>(A, R.invd, b, x, R.z, R.Ap, R.p, hist, ctl, &ri, &ran);
+            if (rc) return rc;
+            if (ran) return finish_resident(ri, info, hhist, noalloc, e0, e1, t0);
+        }
         if (x_zero) {
             HFH_HIP(hipMemcpyAsync(R.r, b, sizeof(T) * n, hipMemcpyDeviceToDevice, s));
             rc = HFH_OK;
@@ -729,19 +780,7 @@ struct PcgWork {
             have_dir = true;
             prev_rz = h.beta;
         }
-        if (hhist && h.iter >= 0) {
-            if (noalloc) {
-                // through the context's 256 pinned result slots, a piece at a time
-                for (int k = 0; k <= h.iter; k += 256) {
-                    const int m = std::min(256, h.iter + 1 - k);
-                    HFH_HIP(hipMemcpyAsync(c->host_res, hist + k, sizeof(double) * m, hipMemcpyDeviceToHost, s));
-                    HFH_HIP(hipStreamSynchronize(s));
-                    std::memcpy(hhist + k, c->host_res, sizeof(double) * m);
-                }
-            } else {
-                HFH_HIP(hipMemcpy(hhist, hist, sizeof(double) * (h.iter + 1), hipMemcpyDeviceToHost));
-            }
-        }
+        if (hhist && h.iter >= 0 && (rc = fetch_hist(hhist, h.iter + 1, noalloc))) return rc;
         if (info) {
             info->iters = h.iter;
             info->state = h.state;

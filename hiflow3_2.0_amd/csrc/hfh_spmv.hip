@@ -890,8 +890,27 @@ static void free_lds_copy(hfh_csr *A) {
 static int round8(long long g) { return static_cast<int>(g >= kNumXcd ? (g + kNumXcd - 1) / kNumXcd * kNumXcd : std::max(g, 1LL)); }
 
 // Configures the SpMV kernel of A (host row pointer in A->h_row).
+// The shape the resident CG needs: the longest row and how far the columns
+// (ascending) reach below and above their row.
+static void row_shape(hfh_csr *A) {
+    A->shape_len = A->shape_lo = A->shape_hi = 0;
+    if (A->nrow != A->ncol || A->nrow > kResidentRows || A->nnz == 0) return;
+    int len = 0, lo = 0, hi = 0;
+    for (int i = 0; i < A->nrow; ++i) {
+        const int j0 = A->h_row[i], j1 = A->h_row[i + 1];
+        if (j1 == j0) continue;
+        len = std::max(len, j1 - j0);
+        lo = std::max(lo, i - A->h_col[j0]);
+        hi = std::max(hi, A->h_col[j1 - 1] - i);
+    }
+    A->shape_len = len;
+    A->shape_lo = lo;
+    A->shape_hi = hi;
+}
+
 int spmv_configure(hfh_csr *A, int algo, int p1, int p2) {
     const int n = A->nrow;
+    row_shape(A);
     // buffers of the previous configuration may still be read by queued work
     HFH_HIP(hipStreamSynchronize(A->ctx->stream));
     if ((algo == HFH_SPMV_SELL || algo == HFH_SPMV_SELL_DICT || algo == HFH_SPMV_SELL_PAIRS ||

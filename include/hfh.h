@@ -331,7 +331,11 @@ typedef struct {
 /* CG<LAD>::SolvePrecond / SolveNoPrecond (linear_solver/cg.cc:84-248) with
  * the scalars kept on the device and the loop launched in chunks; same
  * iterates and stopping test as the reference.  P may be NULL (no
- * preconditioning), Jacobi or MC-SGS.  Returns HFH_OK on convergence,
+ * preconditioning), Jacobi or MC-SGS.  With Jacobi or no preconditioner, an
+ * automatic SpMV layout, at most 28 entries per row and a system that fits on
+ * the chip (up to 524,288 rows of up to 9 entries, 262,144 otherwise; columns
+ * within about 10,000 rows in FP64), the whole solve is one cooperative
+ * launch (HFH_ERR_HIP if one of its bounded waits gave up).  Returns HFH_OK on convergence,
  * HFH_ERR_NOT_CONVERGED on maxits/divergence (info is filled either way).
  * An empty system (n = 0) returns at once: 0 iterations, residual 0,
  * state HFH_SUCCESS_ABS (the same holds for GMRES and defect correction).
