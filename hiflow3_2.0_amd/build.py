@@ -21,7 +21,7 @@ LMP_LIB = os.path.join(HERE, "libhflmp.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("HFH_ARCH", "gfx950")
 
-HIP_SOURCES = ["hfh_core.hip", "hfh_spmv.hip", "hfh_prec.hip", "hfh_pencil.hip", "hfh_krylov.hip", "hfh_cgres.hip",
+HIP_SOURCES = ["hfh_core.hip", "hfh_spmv.hip", "hfh_pattern.hip", "hfh_prec.hip", "hfh_pencil.hip", "hfh_krylov.hip", "hfh_cgres.hip",
                "hfh_batch.hip", "hfh_jacobi.hip", "hfh_analysis.hip", "hfh_assemble.hip", "hfh_vecops.hip", "hfh_matops.hip"]
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",

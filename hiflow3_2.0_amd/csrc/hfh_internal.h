@@ -104,6 +104,20 @@ struct hfh_csr {
     int *sx_cid = nullptr;     // chunk ids (x index / sx_chunk)
     int sx_chunk = 0;          // elements per chunk (16)
     int sx_img = 0;            // largest image of a slice (chunks * sx_chunk)
+    // Matrices of a few distinct (offset, value) pairs (hfh_pattern.hip), on
+    // top of an automatically chosen SELL layout of one wave per slice
+    bool pt_want = false;          // the layout was chosen automatically
+    bool pt_scanned = false;       // pt_rows is up to date with the structure
+    std::vector<int> pt_rows;      // sample rows of every pattern of offsets (empty: too many)
+    int pt_pairs = 0;              // pairs (0: the values do not repeat)
+    int pt_omin = 0, pt_omax = 0;  // smallest and largest offset
+    int pt_ngroups = 0;            // runs of up to three neighbouring offsets
+    bool pt_tri = false;           // all of three
+    void *pt_block = nullptr;      // device memory of the arrays below
+    std::vector<char> pt_lists;    // the runs and the pairs' values, the kernel's argument
+    int *pt_offs = nullptr;        // offsets of the pairs, ascending
+    unsigned *pt_set = nullptr;    // [nrow] the pairs of each row, one bit each
+    int *pt_partial = nullptr;     // [nslice] some row of the slice lacks a pair
     int *diag = nullptr;   // diagonal position per row
     // longest row and how far its columns reach below / above the row, of
     // square matrices small enough for the resident CG (else shape_len 0)
@@ -278,6 +292,14 @@ int spmv_sell_fill(hfh_csr *A);
 int spmv_refresh_structure(hfh_csr *A);
 int spmv_launch_ex(const hfh_csr *A, const void *x, void *y, int mode, const void *w, double *part,
                    const int *done);
+// SpMV by (offset, value) pairs (hfh_pattern.hip): pattern_fill looks at the
+// structure and the values (A->pt_pairs 0 where they do not qualify; waits
+// for the stream), pattern_free forgets them, pattern_spmv launches (as
+// spmv_launch_ex, A->nwg workgroups and partials of the same rows as the SELL
+// kernels).
+int pattern_fill(hfh_csr *A);
+void pattern_free(hfh_csr *A);
+int pattern_spmv(const hfh_csr *A, const void *x, void *y, int mode, const void *w, double *part, const int *done);
 // One Jacobi step xn = update(b - sum_{j != r} a_rj x_j) over the LDS-staged
 // or the dictionary-coded SELL copy (A->spmv_algo HFH_SPMV_SELL_LDS or
 // HFH_SPMV_SELL_DICT); T is A's value type.

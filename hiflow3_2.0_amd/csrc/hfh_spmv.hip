@@ -924,6 +924,8 @@ int spmv_configure(hfh_csr *A, int algo, int p1, int p2) {
     A->sd_wptr = nullptr;
     A->sd_ndict = 0;
     free_lds_copy(A);
+    pattern_free(A);
+    const bool automatic = algo == 0;
     const double mean = n ? static_cast<double>(A->nnz) / n : 0.0;
     // layout taken when the LDS-staged copy does not fit
     int fb_algo = HFH_SPMV_SELL_PAIRS, fb_p1 = 1;
@@ -1159,6 +1161,8 @@ int spmv_configure(hfh_csr *A, int algo, int p1, int p2) {
         set_error("spmv: unknown algorithm %d", algo);
         return HFH_ERR_INVALID;
     }
+    // the SELL layouts' slices: one wave each, kBlock / 64 per workgroup
+    A->pt_want = automatic && A->spmv_algo != HFH_SPMV_STREAM;
     return HFH_OK;
 }
 
@@ -1289,12 +1293,13 @@ int spmv_sell_fill(hfh_csr *A) {
     int rc = launch_check("k_csr_to_sell");
     if (rc) return rc;
     A->sell_dirty = false;
-    return HFH_OK;
+    return pattern_fill(A);
 }
 
 int spmv_launch_ex(const hfh_csr *A, const void *x, void *y, int mode, const void *w, double *part,
                    const int *done) {
     if (A->nrow == 0) return HFH_OK;
+    if (A->pt_pairs > 0) return pattern_spmv(A, x, y, mode, w, part, done);
     const bool dot = w != nullptr;
     if (A->dtype == HFH_F64) {
         if (mode == 0 && !dot) launch_t<double, false, false>(A, x, y, w, part, done);
@@ -1359,6 +1364,7 @@ extern "C" int hfh_csr_destroy(hfh_csr *A) {
     if (A->sd_code) (void)hipFree(A->sd_code);
     if (A->sd_wptr) (void)hipFree(A->sd_wptr);
     free_lds_copy(A);
+    pattern_free(A);
     delete A;
     return HFH_OK;
 }

@@ -125,6 +125,7 @@ HIP_API = {
     "hfh_csr_invdiag": (_i, [_vp, _vp]),
     "hfh_csr_set_spmv": (_i, [_vp, _i, _i, _i]),
     "hfh_csr_get_spmv": (_i, [_vp, _P(_i), _P(_i)]),
+    "hfh_csr_pattern_pairs": (_i, [_vp, _P(_i)]),
     "hfh_jacobi_create": (_i, [_vp, _P(_vp)]),
     "hfh_sgs_create": (_i, [_vp, _i, _vp, _vp, _i, _vp, _vp, _P(_vp)]),
     "hfh_mcsgs_create": (_i, [_vp, _i, _vp, _d, _P(_vp)]),
@@ -500,6 +501,12 @@ class CsrMatrix:
         a, p1 = C.c_int(), C.c_int()
         _ck(hip().hfh_csr_get_spmv(self.h, C.byref(a), C.byref(p1)))
         return a.value, p1.value
+
+    def pattern_pairs(self):
+        """(offset, value) pairs the SpMV runs from (0: the layout of get_spmv)."""
+        k = C.c_int()
+        _ck(hip().hfh_csr_pattern_pairs(self.h, C.byref(k)))
+        return k.value
 
     def set_spmv(self, algo, param1=0, param2=0):
         """Select the SpMV kernel (SPMV_AUTO / SPMV_STREAM / SPMV_VECTOR)."""

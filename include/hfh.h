@@ -205,6 +205,12 @@ enum hfh_spmv_algo { HFH_SPMV_AUTO = 0, HFH_SPMV_STREAM = 1, HFH_SPMV_VECTOR = 2
 int hfh_csr_set_spmv(hfh_csr *A, int algo, int param1, int param2);
 /* the SpMV layout in use (after the automatic choice or a fallback) */
 int hfh_csr_get_spmv(const hfh_csr *A, int *algo, int *param1);
+/* (column offset, value) pairs the matrix consists of, when the automatic
+ * choice found at most 32 of them and the SpMV runs from that list and one
+ * bit set per row (constant-coefficient stencils; bit-identical like SELL);
+ * else 0 and the layout of hfh_csr_get_spmv runs.  Looked at again whenever
+ * the values change. */
+int hfh_csr_pattern_pairs(const hfh_csr *A, int *pairs);
 /* extract_invdiagelements over all rows (lmatrix_csr_cpu.cc:2414-2432) */
 int hfh_csr_invdiag(const hfh_csr *A, hfh_vec *invd);
 /* extract_diagelements / extract_invdiagelements over rows [start, end)
