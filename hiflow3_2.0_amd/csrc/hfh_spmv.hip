@@ -356,15 +356,15 @@ __global__ __launch_bounds__(kBlock) void k_spmv_sellp(
 // last pair, so every load stays in the slice).  Row sums as k_spmv_sellp
 // (ascending slots, uncontracted), so rows agree bit for bit with the CPU
 // loop.  JAC 1 / 2: a Jacobi step (normal / damped) -- entries whose code is
-// the row's diagonal code are skipped and xn_r = jacobi_update(...) is
-// stored instead of the row sum.  xal: x is 16-byte aligned.
+// the row's diagonal code give its 1 / a_rr instead of a product, and xn_r =
+// jacobi_update(...) is stored instead of the row sum.  xal: x is 16-byte aligned.
 template <typename T, bool ADD, bool DOT, int JAC, int CH, int IMG>
 __global__ __launch_bounds__(kBlock) void k_spmv_sellx(
     int nrow, int ncol, int nslice, const int *__restrict__ sptr, const int *__restrict__ rlen,
     const unsigned short *__restrict__ code, const T *__restrict__ sval, const int *__restrict__ cptr,
     const int *__restrict__ cid, int img, int xal, const T *__restrict__ x, T *__restrict__ y,
     const T *__restrict__ w, double *part, const int *__restrict__ done, const unsigned short *__restrict__ dcode,
-    const T *__restrict__ b, const T *__restrict__ invd, T jw, T jomw) {
+    const T *__restrict__ b, T jw, T jomw) {
     typedef typename Pair<T>::type T2;
     typedef typename V16<T>::type TV;
     constexpr int WV = V16<T>::W;              // elements of a 16-byte piece
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_sellx(
         // order: only the compiler has to keep them in program order
         __builtin_amdgcn_wave_barrier();
         asm volatile("" ::: "memory");
-        T acc = 0;
+        T acc = 0, d = 0;   // d: Jacobi, the row's diagonal value
         for (int q = 0; q < Q; ++q) {
             const unsigned cq = cw;
             const T2 vq = v;
@@ -443,14 +443,17 @@ __global__ __launch_bounds__(kBlock) void k_spmv_sellx(
             const int k = 2 * q;
             if (k < len && (!JAC || ka != dc)) acc = add_rn(acc, mul_rn(static_cast<T>(vq.x), xa));
             if (k + 1 < len && (!JAC || kb != dc)) acc = add_rn(acc, mul_rn(static_cast<T>(vq.y), xb));
+            if (JAC && k < len && ka == dc) d = vq.x;
+            if (JAC && k + 1 < len && kb == dc) d = vq.y;
         }
         if (L & 1) {
             const T xt = xs[ct];
             if (2 * Q < len && (!JAC || ct != dc)) acc = add_rn(acc, mul_rn(vt, xt));
+            if (JAC && 2 * Q < len && ct == dc) d = vt;
         }
         if (r < nrow) {
             if (JAC) {
-                y[r] = jacobi_update<T, JAC == 2>(acc, x[r], b[r], invd[r], jw, jomw);
+                y[r] = jacobi_update<T, JAC == 2>(acc, x[r], b[r], dc != 0xffffu ? inverse(d) : T(0), jw, jomw);
             } else {
                 if (ADD) acc = y[r] + acc;
                 y[r] = acc;
@@ -488,8 +491,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_selld(
     int nrow, int ncol, int nslice, const int *__restrict__ sptr, const int *__restrict__ wptr,
     const unsigned *__restrict__ codes, const int *__restrict__ gdict, int ndict,
     const T *__restrict__ sval, const T *__restrict__ x, T *__restrict__ y, const T *__restrict__ w, double *part,
-    const int *__restrict__ done, unsigned code0, const T *__restrict__ b, const T *__restrict__ invd, T jw,
-    T jomw) {
+    const int *__restrict__ done, unsigned code0, const T *__restrict__ b, T jw, T jomw) {
     if (done && *done) return;
     __shared__ int dict[256];
     __shared__ double shd[kBlock / 64];
@@ -503,7 +505,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv_selld(
             const int vbase = sptr[s], L = (sptr[s + 1] - vbase) >> 6, W = (L + 3) >> 2;   // slots, code words
             const int cbase = wptr[s];
             const int r = s * 64 + lane;
-            T acc = 0;
+            T acc = 0, d = 0;        // d: Jacobi, the row's diagonal value, if it has one
+            bool has = false;
             for (int k = 0; k < W; k += UW) {
                 unsigned cw[UW];
                 T v[UW][4], xv[UW][4];
@@ -528,11 +531,15 @@ __global__ __launch_bounds__(kBlock) void k_spmv_selld(
                         const unsigned cd = (cw[u] >> (8 * t)) & 255u;
                         if (k + u < W && cd != kPadCode && (!JAC || cd != code0))
                             acc = add_rn(acc, mul_rn(v[u][t], xv[u][t]));
+                        if (JAC && cd == code0) {
+                            d = v[u][t];
+                            has = true;
+                        }
                     }
             }
             if (r < nrow) {
                 if (JAC) {
-                    y[r] = jacobi_update<T, JAC == 2>(acc, x[r], b[r], invd[r], jw, jomw);
+                    y[r] = jacobi_update<T, JAC == 2>(acc, x[r], b[r], has ? inverse(d) : T(0), jw, jomw);
                 } else {
                     if (ADD) acc = y[r] + acc;
                     y[r] = acc;
@@ -573,7 +580,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv_selld(
         for (; s < nslice; s += stride) {
             const int vbase = nvb, L = nL, W = nW, cbase = ncb;   // slots, code words
             const int r = s * 64 + lane;
-            T acc = 0;
+            T acc = 0, d = 0;        // d: Jacobi, the row's diagonal value, if it has one
+            bool has = false;
             for (int k = 0; k < W; k += UW) {
                 unsigned cw[UW];
                 T v[UW][4], xv[UW][4];
@@ -600,12 +608,16 @@ __global__ __launch_bounds__(kBlock) void k_spmv_selld(
                         const unsigned cd = (cw[u] >> (8 * t)) & 255u;
                         if (k + u < W && cd != kPadCode && (!JAC || cd != code0))
                             acc = add_rn(acc, mul_rn(v[u][t], xv[u][t]));
+                        if (JAC && cd == code0) {
+                            d = v[u][t];
+                            has = true;
+                        }
                     }
             }
             if (W == 0 && s + stride < nslice) fetch(s + stride);   // an empty slice ran no step
             if (r < nrow) {
                 if (JAC) {
-                    y[r] = jacobi_update<T, JAC == 2>(acc, x[r], b[r], invd[r], jw, jomw);
+                    y[r] = jacobi_update<T, JAC == 2>(acc, x[r], b[r], has ? inverse(d) : T(0), jw, jomw);
                 } else {
                     if (ADD) acc = y[r] + acc;
                     y[r] = acc;
@@ -1169,64 +1181,66 @@ int spmv_configure(hfh_csr *A, int algo, int p1, int p2) {
 // The LDS-staged kernel with the image sized to the matrix's largest chunk list.
 template <typename T, bool ADD, bool DOT, int JAC, int CH>
 static void lds_launch_img(const hfh_csr *A, dim3 g, hipStream_t s, int xal, const T *x, T *y, const T *w, double *part,
-                           const int *done, const T *b, const T *invd, T jw, T jomw) {
+                           const int *done, const T *b, T jw, T jomw) {
     const dim3 bl(kBlock);
     const T *sv = static_cast<const T *>(A->sl_val);
     const size_t lds = sizeof(T) * (kBlock / 64) * static_cast<size_t>(A->sx_img);
     if (A->sx_img <= 256)
-        hipLaunchKernelGGL((k_spmv_sellx<T, ADD, DOT, JAC, CH, 256>), g, bl, lds, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sl_len, A->sx_code, sv, A->sx_cptr, A->sx_cid, A->sx_img, xal, x, y, w, part, done, A->sx_dcode, b, invd, jw, jomw);
+        hipLaunchKernelGGL((k_spmv_sellx<T, ADD, DOT, JAC, CH, 256>), g, bl, lds, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sl_len, A->sx_code, sv, A->sx_cptr, A->sx_cid, A->sx_img, xal, x, y, w, part, done, A->sx_dcode, b, jw, jomw);
     else if (A->sx_img <= 512)
-        hipLaunchKernelGGL((k_spmv_sellx<T, ADD, DOT, JAC, CH, 512>), g, bl, lds, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sl_len, A->sx_code, sv, A->sx_cptr, A->sx_cid, A->sx_img, xal, x, y, w, part, done, A->sx_dcode, b, invd, jw, jomw);
+        hipLaunchKernelGGL((k_spmv_sellx<T, ADD, DOT, JAC, CH, 512>), g, bl, lds, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sl_len, A->sx_code, sv, A->sx_cptr, A->sx_cid, A->sx_img, xal, x, y, w, part, done, A->sx_dcode, b, jw, jomw);
     else if (A->sx_img <= 768)
-        hipLaunchKernelGGL((k_spmv_sellx<T, ADD, DOT, JAC, CH, 768>), g, bl, lds, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sl_len, A->sx_code, sv, A->sx_cptr, A->sx_cid, A->sx_img, xal, x, y, w, part, done, A->sx_dcode, b, invd, jw, jomw);
+        hipLaunchKernelGGL((k_spmv_sellx<T, ADD, DOT, JAC, CH, 768>), g, bl, lds, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sl_len, A->sx_code, sv, A->sx_cptr, A->sx_cid, A->sx_img, xal, x, y, w, part, done, A->sx_dcode, b, jw, jomw);
     else
-        hipLaunchKernelGGL((k_spmv_sellx<T, ADD, DOT, JAC, CH, kLdsMaxImage>), g, bl, lds, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sl_len, A->sx_code, sv, A->sx_cptr, A->sx_cid, A->sx_img, xal, x, y, w, part, done, A->sx_dcode, b, invd, jw, jomw);
+        hipLaunchKernelGGL((k_spmv_sellx<T, ADD, DOT, JAC, CH, kLdsMaxImage>), g, bl, lds, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sl_len, A->sx_code, sv, A->sx_cptr, A->sx_cid, A->sx_img, xal, x, y, w, part, done, A->sx_dcode, b, jw, jomw);
 }
 
 template <typename T, bool ADD, bool DOT, int JAC>
 static void lds_launch(const hfh_csr *A, int nwg, const T *x, T *y, const T *w, double *part, const int *done,
-                       const T *b, const T *invd, T jw, T jomw) {
+                       const T *b, T jw, T jomw) {
     hipStream_t s = A->ctx->stream;
     const dim3 g(nwg);
     const int xal = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-    lds_launch_img<T, ADD, DOT, JAC, kLdsChunk>(A, g, s, xal, x, y, w, part, done, b, invd, jw, jomw);
+    lds_launch_img<T, ADD, DOT, JAC, kLdsChunk>(A, g, s, xal, x, y, w, part, done, b, jw, jomw);
 }
 
 // The dictionary-coded kernel; code0 is the code of offset 0 (the diagonal).
 template <typename T, bool ADD, bool DOT, int JAC>
 static void dict_launch(const hfh_csr *A, int nwg, const T *x, T *y, const T *w, double *part, const int *done,
-                        const T *b, const T *invd, T jw, T jomw) {
+                        const T *b, T jw, T jomw) {
     hipStream_t s = A->ctx->stream;
     const dim3 g(nwg), bl(kBlock);
     const T *sv = static_cast<const T *>(A->sl_val);
     const unsigned code0 = static_cast<unsigned>(A->sd_code0);
     if (A->spmv_p1 == 2)
-        hipLaunchKernelGGL((k_spmv_selld<T, ADD, DOT, 2, JAC>), g, bl, 0, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sd_wptr, A->sd_code, A->sd_dict, A->sd_ndict, sv, x, y, w, part, done, code0, b, invd, jw, jomw);
+        hipLaunchKernelGGL((k_spmv_selld<T, ADD, DOT, 2, JAC>), g, bl, 0, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sd_wptr, A->sd_code, A->sd_dict, A->sd_ndict, sv, x, y, w, part, done, code0, b, jw, jomw);
     else
-        hipLaunchKernelGGL((k_spmv_selld<T, ADD, DOT, 1, JAC>), g, bl, 0, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sd_wptr, A->sd_code, A->sd_dict, A->sd_ndict, sv, x, y, w, part, done, code0, b, invd, jw, jomw);
+        hipLaunchKernelGGL((k_spmv_selld<T, ADD, DOT, 1, JAC>), g, bl, 0, s, A->nrow, A->ncol, A->nslice, A->sl_ptr, A->sd_wptr, A->sd_code, A->sd_dict, A->sd_ndict, sv, x, y, w, part, done, code0, b, jw, jomw);
 }
 
 template <typename T>
-int spmv_coded_jacobi(const hfh_csr *A, const T *x, T *xn, const T *b, const T *invd, bool damped, T w, T omw) {
+int spmv_coded_jacobi(const hfh_csr *A, const T *x, T *xn, const T *b, bool damped, T w, T omw) {
     const bool lds = A->spmv_algo == HFH_SPMV_SELL_LDS;
     HFH_CHECK(lds || A->spmv_algo == HFH_SPMV_SELL_DICT, HFH_ERR_INVALID,
               "spmv_coded_jacobi: matrix has no LDS-staged or dictionary-coded copy");
     if (A->nrow == 0) return HFH_OK;
-    const int need = std::max((A->nslice + kBlock / 64 - 1) / (kBlock / 64), 1);
+    int need = std::max((A->nslice + kBlock / 64 - 1) / (kBlock / 64), 1);
+    // FP32 dictionary rows: the SpMV's capped grid, whose waves look ahead over
+    // several slices (three steps on a 141 x 118 x 103 7-point grid: 72 us a
+    // call; 16 workgroups per CU 77 us, one slice per wave 79 us)
+    if (!lds && kDictCappedGrid<T>) need = std::min(need, std::max(A->ctx->num_cu, 1) * 8);
     if (lds && damped)
-        lds_launch<T, false, false, 2>(A, need, x, xn, nullptr, nullptr, nullptr, b, invd, w, omw);
+        lds_launch<T, false, false, 2>(A, need, x, xn, nullptr, nullptr, nullptr, b, w, omw);
     else if (lds)
-        lds_launch<T, false, false, 1>(A, need, x, xn, nullptr, nullptr, nullptr, b, invd, w, omw);
+        lds_launch<T, false, false, 1>(A, need, x, xn, nullptr, nullptr, nullptr, b, w, omw);
     else if (damped)
-        dict_launch<T, false, false, 2>(A, need, x, xn, nullptr, nullptr, nullptr, b, invd, w, omw);
+        dict_launch<T, false, false, 2>(A, need, x, xn, nullptr, nullptr, nullptr, b, w, omw);
     else
-        dict_launch<T, false, false, 1>(A, need, x, xn, nullptr, nullptr, nullptr, b, invd, w, omw);
+        dict_launch<T, false, false, 1>(A, need, x, xn, nullptr, nullptr, nullptr, b, w, omw);
     return launch_check(lds ? "k_spmv_sellx (Jacobi)" : "k_spmv_selld (Jacobi)");
 }
-template int spmv_coded_jacobi<double>(const hfh_csr *, const double *, double *, const double *, const double *,
-                                       bool, double, double);
-template int spmv_coded_jacobi<float>(const hfh_csr *, const float *, float *, const float *, const float *, bool,
-                                      float, float);
+template int spmv_coded_jacobi<double>(const hfh_csr *, const double *, double *, const double *, bool, double, double);
+template int spmv_coded_jacobi<float>(const hfh_csr *, const float *, float *, const float *, bool, float, float);
 
 template <typename T, bool ADD, bool DOT>
 static void launch_t(const hfh_csr *A, const void *x, void *y, const void *w, double *part, const int *done) {
@@ -1235,14 +1249,14 @@ static void launch_t(const hfh_csr *A, const void *x, void *y, const void *w, do
     const T *xv = (const T *)x, *wv = (const T *)w, *val = (const T *)A->val;
     T *yv = (T *)y;
     if (A->spmv_algo == HFH_SPMV_SELL_LDS) {
-        lds_launch<T, ADD, DOT, 0>(A, A->nwg, xv, yv, wv, part, done, nullptr, nullptr, T(0), T(0));
+        lds_launch<T, ADD, DOT, 0>(A, A->nwg, xv, yv, wv, part, done, nullptr, T(0), T(0));
     } else if (A->spmv_algo == HFH_SPMV_SELL_PAIRS) {
         if (A->spmv_p1 == 2)
             hipLaunchKernelGGL((k_spmv_sellp<T, ADD, DOT, 2>), g, bl, 0, s, A->nrow, A->nslice, A->sl_ptr, A->sl_len, A->sl_col, (const T *)A->sl_val, xv, yv, wv, part, done);
         else
             hipLaunchKernelGGL((k_spmv_sellp<T, ADD, DOT, 1>), g, bl, 0, s, A->nrow, A->nslice, A->sl_ptr, A->sl_len, A->sl_col, (const T *)A->sl_val, xv, yv, wv, part, done);
     } else if (A->spmv_algo == HFH_SPMV_SELL_DICT) {
-        dict_launch<T, ADD, DOT, 0>(A, A->nwg, xv, yv, wv, part, done, nullptr, nullptr, T(0), T(0));
+        dict_launch<T, ADD, DOT, 0>(A, A->nwg, xv, yv, wv, part, done, nullptr, T(0), T(0));
     } else if (A->spmv_algo == HFH_SPMV_SELL) {
         switch (A->spmv_p1) {
         case 2: hipLaunchKernelGGL((k_spmv_sell<T, ADD, DOT, 2>), g, bl, 0, s, A->nrow, A->nslice, A->sl_ptr, A->sl_len, A->sl_col, (const T *)A->sl_val, xv, yv, wv, part, done); break;

@@ -166,3 +166,38 @@ def test_swapped_matrix_refused_by_ordered_setups(pkg, ctx):
     X, Y = pkg.Vector(ctx, np.ones(len(row) - 1)), pkg.Vector(ctx, len(row) - 1)
     P.apply(X, Y)
     assert np.all(np.isfinite(Y.numpy()))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("mode", ["JACOBI_SMOOTH_NORMAL", "JACOBI_SMOOTH_DAMPED"])
+def test_smoother_step_counts(pkg, ctx, mode, dtype):
+    """m steps in one call equal m calls of one step, bit for bit, for odd and
+    even m and growing and shrinking systems (the work space is kept between
+    calls); rows without a diagonal keep an inverse of 0."""
+    rng = np.random.default_rng(3)
+    for n in (200, 40000, 777):
+        i = np.arange(n)
+        row = np.concatenate([[0], np.cumsum(np.where((i == 0) | (i == n - 1), 2, 3) - (i % 50 == 7))]).astype(np.int32)
+        c = np.stack([i - 1, i, i + 1], 1)
+        keep = (c >= 0) & (c < n)
+        keep[i % 50 == 7, 1] = False
+        v = rng.uniform(-1, 1, c.shape)
+        v[:, 1] = rng.uniform(3, 4, n)
+        A = pkg.CsrMatrix(ctx, row, c[keep].astype(np.int32), v[keep].astype(dtype))
+        b, x0 = pkg.Vector(ctx, rng.standard_normal(n), dtype), rng.standard_normal(n)
+        one = pkg.Vector(ctx, x0, dtype)
+        for m in range(1, 6):
+            pkg.jacobi(A, b, one, mode=getattr(pkg, mode), w=0.7, inner_iter=1, smooth_iter=1)
+            x = pkg.Vector(ctx, x0, dtype)
+            pkg.jacobi(A, b, x, mode=getattr(pkg, mode), w=0.7, inner_iter=m, smooth_iter=1)
+            assert np.array_equal(x.numpy(), one.numpy())
+        D = np.zeros((n, 3))
+        D[keep] = v[keep].astype(dtype)
+        inv = np.where(D[:, 1] != 0, 1 / np.where(D[:, 1] != 0, D[:, 1], 1), 0)
+        y = x0.astype(dtype).astype(np.float64)
+        for _ in range(5):
+            s = D[:, 0] * np.concatenate([[0], y[:-1]]) + D[:, 2] * np.concatenate([y[1:], [0]])
+            new = (b.numpy().astype(np.float64) - s) * inv
+            y = new if mode == "JACOBI_SMOOTH_NORMAL" else 0.3 * y + 0.7 * new
+        # each step rounds about 6 operations on values near |y|; 5 steps
+        assert np.max(np.abs(x.numpy() - y)) <= 60 * np.finfo(dtype).eps * max(1.0, np.max(np.abs(y)))
