@@ -30,6 +30,7 @@ constexpr int kRedBlocks = 1024;     // max partials per reduction
 // slot (a slot past its row's length), so kernels need no row lengths;
 // dictionaries therefore hold at most 255 offsets
 constexpr unsigned kPadCode = 255;
+constexpr int kHostDot = 255;        // word of host_res that such a dot's result arrives in
 constexpr int kNumXcd = 8;           // MI355X: 8 accelerator complex dies
 // Size of the per-device static array that the allocation-free CG
 // (hfh_pcg_solve_noalloc) works in: FP64 systems up to 2,096,000 rows.
@@ -57,6 +58,7 @@ struct hfh_ctx {
     // reduction scratch: partials[kRedBlocks * 8] doubles, then result slots
     double *red = nullptr;            // device
     double *host_res = nullptr;       // pinned host mirror for results
+    unsigned long long *dot_slots = nullptr;   // partials of dots that the host waits for (in red)
     hfh::Timing timing;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int live = 0;                     // vectors, matrices and preconditioners created on the context
