@@ -33,9 +33,12 @@
 //
 // Measured (apply, both sweeps, FP64; blocks -> pencils): upwind 128^3 ILU(0)
 // 480 -> 267 us, SGS 529 -> 284 us; 2D 701 x 509 SGS 896 -> 427 us; 40^3 SGS
-// 136 -> 86 us; 16^3 51 -> 35 us; 64 x 64 90 -> 49 us.  A step takes about
-// 150 ns (LDS write to read, then the chain of products and sums) and a hop
-// to the next pencil about 2 us on top of its skew.
+// 136 -> 86 us; 16^3 51 -> 35 us; 64 x 64 90 -> 49 us.  A step took about 150
+// ns and a hop to the next pencil about 2 us on top of its skew.  The step is
+// bound by what a lone wave issues: a dependent FP64 operation 6 to 7 cycles, an
+// LDS write and read back 66, a lane shift of a double 31, a branch on lanes'
+// values 70.  Without branches in the steps, with lane shifts instead of LDS
+// in 2D and plain value loads, 2D 701 x 509 SGS takes 383 us.
 #include "hfh_internal.h"
 
 #include <algorithm>
@@ -44,7 +47,12 @@ namespace hfh {
 
 namespace {
 
-constexpr int kAhead = 4;       // groups of 4 steps whose operands are in flight
+// Groups of 4 steps whose operands are in flight (upwind 128^3 GMRES + ILU(0) /
+// 2D 701 x 509 SGS: 4 groups 94.1 ms / 384 us, 6 93.9 / 383, 8 93.4 / 411).
+// Both forms of a group issue the same number of accesses, so that the waits
+// count them exactly: with two 16-byte accesses in place of four inside the
+// lines GMRES took 100 ms.
+constexpr int kAhead = 6;
 constexpr int kSlots = 32;      // steps held in the LDS ring
 constexpr int kPencilSpins = 1 << 20;
 
@@ -72,19 +80,33 @@ template <> struct Bits<float> {
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
-// a / d rounded once, r = RN(1 / d) (see above).  slow: all ones where some
-// diagonal of the matrix lies outside [dlo, dhi], so that every lane then
-// divides plainly; else 0.
+// a / d rounded once, r = RN(1 / d) (see above), where |a| lies in the range
+// of the fast form or a is +0; else `worst` becomes at least Bits<T>::alen and
+// the caller divides plainly.
 template <typename T>
-__device__ __forceinline__ T quotient(T a, T d, T r, unsigned slow) {
+__device__ __forceinline__ T quotient(T a, T d, T r, unsigned &worst) {
     typedef typename Bits<T>::U U;
     T q = mul_rn(a, r);
     q = fma_t(fma_t(-q, d, a), r, q);
     q = fma_t(fma_t(-q, d, a), r, q);
-    const unsigned t = ((Bits<T>::top(a) << 1) - Bits<T>::alo) | slow;
-    const bool ok = t < Bits<T>::alen || (__builtin_bit_cast(U, a) | slow) == 0;
-    if (!__builtin_amdgcn_ballot_w64(!ok)) return q;
-    return ok ? q : a / d;
+    const unsigned t = (Bits<T>::top(a) << 1) - Bits<T>::alo;
+    worst = max(worst, __builtin_bit_cast(U, a) == 0 ? 0u : t);
+    return q;
+}
+
+// The value of the lane below; lane 0 gets `edge`.
+__device__ __forceinline__ unsigned lane_below(unsigned v, unsigned edge) {
+    return __builtin_amdgcn_update_dpp(edge, v, 0x138, 0xf, 0xf, false);   // wave_shr:1
+}
+__device__ __forceinline__ float from_below(float v, float edge) {
+    return __builtin_bit_cast(float, lane_below(__builtin_bit_cast(unsigned, v), __builtin_bit_cast(unsigned, edge)));
+}
+__device__ __forceinline__ double from_below(double v, double edge) {
+    typedef unsigned long long U;
+    const U a = __builtin_bit_cast(U, v), e = __builtin_bit_cast(U, edge);
+    const unsigned lo = lane_below(static_cast<unsigned>(a), static_cast<unsigned>(e));
+    const unsigned hi = lane_below(static_cast<unsigned>(a >> 32), static_cast<unsigned>(e >> 32));
+    return __builtin_bit_cast(double, static_cast<U>(hi) << 32 | lo);
 }
 
 template <typename T>
@@ -93,18 +115,11 @@ __device__ __forceinline__ typename Bits<T>::U face_load(const T *p) {
                              __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Arithmetic results are never the sentinel; a copied NaN could be.
-template <typename T>
-__device__ __forceinline__ void face_store(T *p, T v) {
-    typedef typename Bits<T>::U U;
-    U u = __builtin_bit_cast(U, v);
-    if (u == Bits<T>::sentinel) u |= Bits<T>::quiet;
-    __hip_atomic_store(reinterpret_cast<U *>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Element access with a byte offset checked against the vector's size: a
 // lane outside the grid uses kOutside, reads 0 and stores nothing.
-constexpr unsigned kOutside = 0xFFFFF000u;
+// kOutside + a line's own offset is outside as well: vectors and inboxes are
+// at most 2^31 bytes, a line's offsets below 2^30.
+constexpr unsigned kOutside = 0xC0000000u;
 typedef unsigned U2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ double vec_load(__amdgpu_buffer_rsrc_t b, unsigned off, double) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, off, 0, 0));
@@ -117,6 +132,28 @@ __device__ __forceinline__ void vec_store(__amdgpu_buffer_rsrc_t b, unsigned off
 }
 __device__ __forceinline__ void vec_store(__amdgpu_buffer_rsrc_t b, unsigned off, float v) {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), b, off, 0, 0);
+}
+// A face value, visible to the other CUs (agent scope: sc1), without the
+// branch that an exec-masked store costs.  It is the result of an addition,
+// so never the sentinel: those quiet a signalling NaN.
+constexpr int kAgentScope = 16;
+typedef unsigned U4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void face_store(__amdgpu_buffer_rsrc_t b, unsigned off, double v) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), b, off, 0, kAgentScope);
+}
+__device__ __forceinline__ void face_store(__amdgpu_buffer_rsrc_t b, unsigned off, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), b, off, 0, kAgentScope);
+}
+
+// Four neighbouring face values, the lowest at `off` (aligned to an element).
+__device__ __forceinline__ void face_store4(__amdgpu_buffer_rsrc_t b, unsigned off, const double (&v)[4]) {
+    typedef double D2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, D2{v[0], v[1]}), b, off, 0, kAgentScope);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, D2{v[2], v[3]}), b, off + 16, 0, kAgentScope);
+}
+__device__ __forceinline__ void face_store4(__amdgpu_buffer_rsrc_t b, unsigned off, const float (&v)[4]) {
+    typedef float F4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(U4, F4{v[0], v[1], v[2], v[3]}), b, off, 0, kAgentScope);
 }
 
 // The shape of a sweep's pencils.  Coordinates are the sweep's own: the
@@ -162,7 +199,7 @@ __global__ __launch_bounds__(128) void k_pencil(PencilArgs<T> a) {
     const int ng = a.ng, np = a.npy * a.npz;
     // the other sweep's ticket counter starts its next launch at 0
     if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl[FW ? 32 : 0] = 0;
-    const unsigned slow = DIV && a.ctl[64] != 0 ? ~0u : 0u;
+    const bool slow = DIV && a.ctl[64] != 0;   // some diagonal is outside [dlo, dhi]
     for (;;) {
         // Pencils are taken in dependency order, so the earliest unfinished
         // one never waits for a pencil that no workgroup holds.
@@ -264,22 +301,31 @@ __global__ __launch_bounds__(128) void k_pencil(PencilArgs<T> a) {
             auto at = [&](int s) {
                 return static_cast<unsigned>(x00 + s) < static_cast<unsigned>(a.nx) ? off00 + static_cast<unsigned>(dir * s) : kOutside;
             };
+            const unsigned off0 = valid ? off00 : kOutside;
+            // steps of a group past every line's start and before any one's end
+            auto inside = [&](int gi) { return 4 * gi >= S::SKEW && 4 * gi + 3 < a.nx; };
             const unsigned nbytes = static_cast<unsigned>(static_cast<long long>(a.nx) * a.ny * a.nz * sizeof(T));
             const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(FW ? a.in : a.out), (short)0, nbytes, 0x00027000);
-            const V2 *vbase = reinterpret_cast<const V2 *>(a.val) + static_cast<size_t>(pn) * ng * 2 * K * 64 + lane;
+            const V2 *vbase = reinterpret_cast<const V2 *>(a.val) + static_cast<size_t>(pn) * ng * 2 * K * 64;
             const size_t slab = static_cast<size_t>(4) * ng + 4;
-            T *const yw = a.y + (static_cast<size_t>(pn) * slab + 4) * 64 + lane;
+            // a line outside the grid stores nothing: its results stay 0 there
+            const auto ys = __builtin_amdgcn_make_buffer_rsrc(a.y + static_cast<size_t>(pn) * slab * 64, (short)0,
+                                                              static_cast<unsigned>(slab * 64 * sizeof(T)), 0x00027000);
+            const unsigned yoff = valid ? (4 * 64 + lane) * static_cast<unsigned>(sizeof(T)) : kOutside;
             const T *const yr = a.y + (static_cast<size_t>(rp) * slab + 4 + a.nx + S::SKEW - 1) * 64 + 63 - lane;
             // where this wave's y / z neighbours' results stand in a slot
             const bool yin = yl > 0, zin = zl > 0;
-            const int aB = !valid ? S::ZERO : yin ? lane - 1 : 64 + zl;
+            const int aB = !valid ? S::ZERO : yin ? lane - 1 : 64 + zl;   // 3D
             const int aC = !valid ? S::ZERO : zin ? lane - 8 : 72 + yl;
-            // faces out: lane -> (row of the group, face value) -> the successor's inbox
-            const int frow = lane / H, fe = lane % H;
-            const bool yface = !D3 || fe < 8;
-            const int fsrc = !D3 ? 63 : yface ? 7 + 8 * fe : 56 + fe - 8;
-            const bool fout = frow < 4 && (yface ? J + 1 < a.npy : KK + 1 < a.npz);
-            T *const fdst = a.box + (static_cast<size_t>(yface ? pn + 1 : pn + a.npy) * ng * 4 + frow) * H + fe;
+            // 3D, faces out: lane -> (row of the group, face value) -> the successor's inbox
+            const int frow = lane / 16, fe = lane % 16;
+            const bool yface = fe < 8;
+            const int fsrc = yface ? 7 + 8 * fe : 56 + fe - 8;
+            const auto bs = __builtin_amdgcn_make_buffer_rsrc(a.box, (short)0, static_cast<unsigned>(sizeof(T)) * np * ng * 4 * H, 0x00027000);
+            const unsigned ES = sizeof(T);
+            const unsigned fdst = !D3 ? (lane == 63 && J + 1 < a.npy ? ((pn + 1) * ng * 4 + 1) * ES : kOutside)
+                                : (yface ? J + 1 < a.npy : KK + 1 < a.npz)
+                                    ? (((yface ? pn + 1 : pn + a.npy) * ng * 4 + frow) * H + fe) * ES : kOutside;
             struct Grp {
                 V2 v[2][K];
                 T s[4];
@@ -290,11 +336,14 @@ __global__ __launch_bounds__(128) void k_pencil(PencilArgs<T> a) {
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
 #pragma unroll
-                    for (int k = 0; k < K; ++k) g.v[h][k] = __builtin_nontemporal_load(p + (h * K + k) * 64);
+                    for (int k = 0; k < K; ++k) g.v[h][k] = p[(h * K + k) * 64 + lane];
+                if (!FW) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (FW) g.s[j] = vec_load(rs, at(4 * gi + j), T(0));
-                    else g.s[j] = yr[-(4 * gi + j) * 64];
+                    for (int j = 0; j < 4; ++j) g.s[j] = yr[-(4 * gi + j) * 64];
+                } else {
+                    const bool in = inside(gi);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) g.s[j] = vec_load(rs, in ? off0 + dir * (4 * gi + j) : at(4 * gi + j), T(0));
                 }
             };
             T prev = T(0);
@@ -306,39 +355,62 @@ __global__ __launch_bounds__(128) void k_pencil(PencilArgs<T> a) {
                 asm volatile("" ::: "memory");
                 T *const base = ring + (gi & (kSlots / 4 - 1)) * 4 * SLOT;
                 T *const next = ring + ((gi + 1) & (kSlots / 4 - 1)) * 4 * SLOT;
+                T face[4], res[4], f = T(0);
+                if (!D3) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const T B = base[j * SLOT + aB];
-                    const T C = D3 ? base[j * SLOT + aC] : T(0);
-                    const T A = prev;
-                    const V2(&v)[K] = g.v[j >> 1];
-                    T acc = g.s[j];
-                    if (FW) {
-                        if (D3) acc = add_rn(acc, -mul_rn(C, v[NV - 1][j & 1]));
-                        acc = add_rn(acc, -mul_rn(B, v[1][j & 1]));
-                        acc = add_rn(acc, -mul_rn(A, v[0][j & 1]));
-                    } else {
-                        if (MODE == 1) acc = mul_rn(acc, v[NV][j & 1]);
-                        acc = add_rn(acc, -mul_rn(A, v[0][j & 1]));
-                        acc = add_rn(acc, -mul_rn(B, v[1][j & 1]));
-                        if (D3) acc = add_rn(acc, -mul_rn(C, v[NV - 1][j & 1]));
-                    }
-                    if (DIV) acc = quotient<T>(acc, v[K - 2][j & 1], v[K - 1][j & 1], slow);
-                    // a lane before or past its line holds 0, whatever its neighbours hold
-                    if (edge) acc = at(4 * gi + j) != kOutside ? acc : T(0);
-                    prev = acc;
-                    (j < 3 ? base + (j + 1) * SLOT : next)[lane] = acc;
-                    __builtin_amdgcn_wave_barrier();
-                    if (j == 2) {
-                        // the group's four slots hold steps 4 gi - 1 .. 4 gi + 2
-                        const T f = base[(D3 ? frow : frow & 3) * SLOT + fsrc];
-                        if (fout) face_store(fdst + static_cast<size_t>(gi) * 4 * H, f);
-                    }
-                    if (FW) yw[(4 * gi + j) * 64] = acc;
-                    else vec_store(rs, at(4 * gi + j), acc);
+                    for (int j = 0; j < 4; ++j) face[j] = base[j * SLOT + 64];
                 }
+                const T prev0 = prev;
+                unsigned worst = 0;
+                auto steps = [&](bool plain) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        // 2D: the y neighbour's result from its lane's register
+                        const T B = D3 ? base[j * SLOT + aB] : from_below(prev, face[j]);
+                        const T C = D3 ? base[j * SLOT + aC] : T(0);
+                        const T A = prev;
+                        const V2(&v)[K] = g.v[j >> 1];
+                        T acc = g.s[j];
+                        if (FW) {
+                            if (D3) acc = add_rn(acc, -mul_rn(C, v[NV - 1][j & 1]));
+                            acc = add_rn(acc, -mul_rn(B, v[1][j & 1]));
+                            acc = add_rn(acc, -mul_rn(A, v[0][j & 1]));
+                        } else {
+                            if (MODE == 1) acc = mul_rn(acc, v[NV][j & 1]);
+                            acc = add_rn(acc, -mul_rn(A, v[0][j & 1]));
+                            acc = add_rn(acc, -mul_rn(B, v[1][j & 1]));
+                            if (D3) acc = add_rn(acc, -mul_rn(C, v[NV - 1][j & 1]));
+                        }
+                        if (DIV && plain) acc = acc / v[K - 2][j & 1];
+                        else if (DIV) acc = quotient<T>(acc, v[K - 2][j & 1], v[K - 1][j & 1], worst);
+                        // a lane before or past its line holds 0, whatever its neighbours hold
+                        if (edge) acc = at(4 * gi + j) != kOutside ? acc : T(0);
+                        prev = res[j] = acc;
+                        if (D3) {
+                            (j < 3 ? base + (j + 1) * SLOT : next)[lane] = acc;
+                            __builtin_amdgcn_wave_barrier();
+                            // the group's four slots hold steps 4 gi - 1 .. 4 gi + 2
+                            if (j == 2) f = base[frow * SLOT + fsrc];
+                        }
+                        if (FW) vec_store(ys, yoff + (4 * gi + j) * 64 * ES, acc);
+                        else vec_store(rs, edge ? at(4 * gi + j) : off0 + dir * (4 * gi + j), acc);
+                    }
+                };
+                // A branch on lanes' values costs a step half its time, so the
+                // range of the divisions is looked at once per group, which is
+                // then computed again; its faces leave after that.
+                if (!slow) steps(false);
+                if (DIV && (slow || __builtin_amdgcn_ballot_w64(worst >= Bits<T>::alen))) {
+                    prev = prev0;
+                    steps(true);
+                }
+                if (D3) face_store(bs, fdst + static_cast<unsigned>(gi) * 4 * H * ES, f);
+                // 2D: the inbox rows lie side by side; the last step's row is
+                // row 0 of the next inbox, which nobody reads
+                else face_store4(bs, fdst + 4 * gi * ES, res);
                 asm volatile("" ::: "memory");
-                if (lane == 0) __hip_atomic_store(&s_read, gi + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                // every lane the same value: no branch
+                __hip_atomic_store(&s_read, gi + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             };
 #pragma unroll
             for (int k = 0; k < kAhead; ++k) load(grp[k], k);
@@ -347,8 +419,8 @@ __global__ __launch_bounds__(128) void k_pencil(PencilArgs<T> a) {
                 for (int k = 0; k < kAhead; ++k) {
                     const int gi = g0 + k;
                     if (gi < ng) {
-                        if (4 * gi < S::SKEW || 4 * gi + 3 >= a.nx) group(grp[k], gi, true);
-                        else group(grp[k], gi, false);
+                        if (inside(gi)) group(grp[k], gi, false);
+                        else group(grp[k], gi, true);
                     }
                     load(grp[k], gi + kAhead);
                 }
@@ -508,6 +580,8 @@ int pencil_build(hfh_prec *P, int nx, long long nxy) {
     G.np = G.npy * G.npz;
     // one step past the last lane's: the faces leave one step later
     G.ng = (nx + (d3 ? 15 : 64) + 3) / 4;
+    // offsets within a pencil's inbox, results and values in 32 bits
+    if (4LL * G.ng * (64 * 5) * es >= (1LL << 30)) return HFH_OK;
     // the skew's idle steps must not dominate the value copies
     const long long slots = 256LL * G.np * G.ng;
     if (slots > 4LL * n) return HFH_OK;
