@@ -1021,14 +1021,14 @@ constexpr int kMaxBasis = 256;
 // The whole MGS sweep of one Arnoldi column in one cooperative launch
 // (GMRES::SolveRight's inner loop, gmres.cc:285-510): h_i = w.v_i and
 // w -= h_i v_i for i = 0..j, then h_{j+1} = ||w|| and v_{j+1} = w / h_{j+1},
-// with the same per-element arithmetic as k_mgs and k_norm_scale_into.  Each
-// thread keeps its E elements of w in registers for the whole sweep and
-// loads the next basis vector while a step's sum travels, so a step reads
-// only v_i from memory (k_mgs reads w, v_(i-1) and v_i and writes w).  The
-// step's sum crosses the grid without a fence: every workgroup stores its
-// partial with an agent-scope relaxed atomic store over a signalling-NaN
-// sentinel, then polls all G partials (each value its own flag) and sums
-// them in one fixed order, so every workgroup holds the same h_i.  The
+// the vectors taken two at a time (below).  Each thread keeps its E elements
+// of w in registers for the whole sweep and loads the next pair while a
+// step's sums travel, so a step reads only its vectors from memory (k_mgs
+// reads w, v_(i-1) and v_i and writes w).  The step's sums cross the grid
+// without a fence: every workgroup stores its partials with agent-scope
+// relaxed atomic stores over a signalling-NaN sentinel, then polls all G
+// partials (each value its own flag) and sums them in one fixed order, so
+// every workgroup holds the same h_i.  The
 // partials of the launches alternate between two halves of `slots` (par);
 // each workgroup sets its own slots of the other half back to the sentinel
 // for the next launch.  The launch is cooperative: all G workgroups are
@@ -1038,102 +1038,132 @@ constexpr int kCoopBlock = 1024;
 constexpr int kCoopSpins = 1 << 16;
 constexpr unsigned long long kCoopSentinel = 0x7FF4DEAD5EEDBEEFull;   // exponent all ones, quiet bit clear
 
-// Sum of one step over the grid, valid in every thread: this workgroup's
-// partial (wave trees, then the waves in order) published in slot row[g],
-// then the G partials polled and summed (thread t holds row[t]; wave trees,
-// then the waves in order).
-__device__ __forceinline__ double coop_step_sum(double v, unsigned long long *row, double *sh, double *bc,
-                                                int *fail) {
-    const int G = gridDim.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    v = wave_sum(v);
-    if (lane == 0) sh[wv] = v;
-    __syncthreads();
-    if (tid == 0) {
-        double t = 0;
-        for (int k = 0; k < kCoopBlock / 64; ++k) t += sh[k];
-        __hip_atomic_store(row + blockIdx.x, __builtin_bit_cast(unsigned long long, t), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+// Three sums over the grid at once, valid in every thread: this workgroup's
+// partials (wave sums, then the waves in order) published in slots
+// row[q G + g], then the G partials of each polled and summed (wave sums, then
+// the waves in order).  Publishing copies, so that fewer workgroups poll one,
+// changed nothing here (1, 8 and 16 copies: 92.4, 92.1, 92.3 ms).
+constexpr int kCoopSums = 3;
+
+__device__ __forceinline__ void coop_step_sums(const double (&v)[kCoopSums], unsigned long long *row,
+                                               double (*sh)[kCoopBlock / 64], double (*sh2)[kCoopBlock / 64],
+                                               int *fail, double (&out)[kCoopSums]) {
+    const int G = gridDim.x, Gp = (G + 63) & ~63, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+#pragma unroll
+    for (int q = 0; q < kCoopSums; ++q) {
+        const double t = wave_sum_dpp(v[q]);
+        if (lane == 0) sh[q][wv] = t;
     }
-    double x = 0;
-    if (tid < G) {
-        unsigned long long u = __hip_atomic_load(row + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        int spins = 0;
-        while (u == kCoopSentinel && spins < kCoopSpins) {
-            ++spins;
-            __builtin_amdgcn_s_sleep(1);
-            u = __hip_atomic_load(row + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (tid < kCoopSums) {
+        double t = 0;
+        for (int k = 0; k < kCoopBlock / 64; ++k) t += sh[tid][k];
+        __hip_atomic_store(row + static_cast<long long>(tid) * G + blockIdx.x, __builtin_bit_cast(unsigned long long, t),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const int q = tid / Gp, i = tid - q * Gp;   // whole waves: Gp is a multiple of 64
+    if (q < kCoopSums) {
+        double x = 0;
+        if (i < G) {
+            unsigned long long *slot = row + static_cast<long long>(q) * G + i;
+            unsigned long long u = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            int spins = 0;
+            while (u == kCoopSentinel && spins < kCoopSpins) {
+                ++spins;
+                __builtin_amdgcn_s_sleep(1);
+                u = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            if (u == kCoopSentinel) __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            x = __builtin_bit_cast(double, u);
         }
-        if (u == kCoopSentinel) __hip_atomic_store(fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        x = __builtin_bit_cast(double, u);
+        x = wave_sum_dpp(x);
+        if (lane == 0) sh2[q][i >> 6] = x;
     }
-    __syncthreads();   // sh is reused
-    x = wave_sum(x);
-    if (lane == 0) sh[wv] = x;
     __syncthreads();
-    if (tid == 0) {
+#pragma unroll
+    for (int k = 0; k < kCoopSums; ++k) {
         double t = 0;
-        for (int k = 0; k < (G + 63) / 64; ++k) t += sh[k];
-        *bc = t;
+        for (int w = 0; w < Gp / 64; ++w) t += sh2[k][w];
+        out[k] = t;
     }
-    __syncthreads();
-    return *bc;
 }
 
+// The MGS sweep of column j by pairs of basis vectors, one grid sum each:
+// with s0 = w.v_i, s1 = w.v_{i+1} and g = v_i.v_{i+1} the modified
+// Gram-Schmidt coefficients are h_i = s0 and h_{i+1} = (w - h_i v_i).v_{i+1} =
+// s1 - h_i g.  Between two sums the memory idles while the sum is formed,
+// travels and w is updated, so a sum for two vectors halves that: upwind
+// 128^3 GMRES(30) + ILU(0) 94.5 -> 92.2 ms.  The workgroup's 128 registers
+// per thread hold w and two pairs with a few spilled; 512 threads of 16
+// elements each ran the same.
 template <typename T, int E>
 __global__ __launch_bounds__(kCoopBlock) void k_mgs_coop(int n, const T *__restrict__ w, T *const *__restrict__ V,
                                                          int j, unsigned long long *slots, int nstep, int par,
                                                          double *Hd, int *fail) {
-    __shared__ double sh[kCoopBlock / 64];
-    __shared__ double bc;
+    __shared__ double sh[kCoopSums][kCoopBlock / 64], sh2[kCoopSums][kCoopBlock / 64];
     const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
     const long long span = static_cast<long long>(G) * kCoopBlock;
     const long long i0 = static_cast<long long>(g) * kCoopBlock + tid;
-    if (tid < nstep) slots[(static_cast<long long>(1 - par) * nstep + tid) * G + g] = kCoopSentinel;
-    T wr[E], vr[E], vn[E];
-    {
-        const T *v0 = V[0];
+    const long long per = static_cast<long long>(kCoopSums) * G;   // slots of a step
+    for (int k = tid; k < nstep * kCoopSums; k += kCoopBlock)
+        slots[(1 - par) * nstep * per + static_cast<long long>(k) * G + g] = kCoopSentinel;
+    T wr[E], va[E], vb[E], na[E], nb[E];
+    auto load = [&](int i, T(&v)[E]) {   // basis vector i, or zeros past column j
+        const T *p = V[min(i, j)];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const long long i = i0 + e * span;
-            wr[e] = i < n ? w[i] : static_cast<T>(0);
-            vr[e] = i < n ? v0[i] : static_cast<T>(0);
+            const long long k = i0 + e * span;
+            v[e] = i <= j && k < n ? p[k] : static_cast<T>(0);
+        }
+    };
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const long long i = i0 + e * span;
+        wr[e] = i < n ? w[i] : static_cast<T>(0);
+    }
+    load(0, va);
+    load(1, vb);
+    unsigned long long *row = slots + par * nstep * per;
+    double s[kCoopSums], tot[kCoopSums];
+    for (int i = 0; i <= j; i += 2, row += per) {
+        s[0] = s[1] = s[2] = 0;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            s[0] += static_cast<double>(wr[e]) * static_cast<double>(va[e]);
+            s[1] += static_cast<double>(wr[e]) * static_cast<double>(vb[e]);
+            s[2] += static_cast<double>(va[e]) * static_cast<double>(vb[e]);
+        }
+        // the next pair, loaded while the sums travel
+        load(i + 2, na);
+        load(i + 3, nb);
+        coop_step_sums(s, row, sh, sh2, fail, tot);
+        const T h0 = static_cast<T>(tot[0]);
+        const T h1 = static_cast<T>(tot[1] - static_cast<double>(h0) * tot[2]);
+        if (g == 0 && tid == 0) {
+            Hd[i] = static_cast<double>(h0);
+            if (i < j) Hd[i + 1] = static_cast<double>(h1);
+        }
+        const T m0 = static_cast<T>(-1) * h0, m1 = static_cast<T>(-1) * h1;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            wr[e] += m0 * va[e];
+            wr[e] += m1 * vb[e];
+            va[e] = na[e];
+            vb[e] = nb[e];
         }
     }
-    for (int i = 0; i <= j + 1; ++i) {   // step j + 1: the norm
-        double sum = 0;
+    s[0] = s[1] = s[2] = 0;
 #pragma unroll
-        for (int e = 0; e < E; ++e)
-            sum += static_cast<double>(wr[e]) * static_cast<double>(i <= j ? vr[e] : wr[e]);
-        if (i + 1 <= j) {   // the next basis vector, loaded while the sum travels
-            const T *vnext = V[i + 1];
+    for (int e = 0; e < E; ++e) s[0] += static_cast<double>(wr[e]) * static_cast<double>(wr[e]);
+    coop_step_sums(s, row, sh, sh2, fail, tot);
+    const T hn = static_cast<T>(sqrt(static_cast<double>(static_cast<T>(tot[0]))));
+    if (g == 0 && tid == 0) Hd[j + 1] = static_cast<double>(hn);
+    const T sc = static_cast<T>(1) / hn;
+    T *vj1 = V[j + 1];
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const long long k = i0 + e * span;
-                vn[e] = k < n ? vnext[k] : static_cast<T>(0);
-            }
-        }
-        const double tot = coop_step_sum(sum, slots + (static_cast<long long>(par) * nstep + i) * G, sh, &bc, fail);
-        if (i <= j) {
-            const T hi = static_cast<T>(tot);
-            if (g == 0 && tid == 0) Hd[i] = static_cast<double>(hi);
-            const T mh = static_cast<T>(-1) * hi;
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                wr[e] += mh * vr[e];
-                vr[e] = vn[e];
-            }
-        } else {
-            const T d = static_cast<T>(tot);
-            const T hn = static_cast<T>(sqrt(static_cast<double>(d)));
-            if (g == 0 && tid == 0) Hd[j + 1] = static_cast<double>(hn);
-            const T sc = static_cast<T>(1) / hn;
-            T *vj1 = V[j + 1];
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const long long k = i0 + e * span;
-                if (k < n) vj1[k] = wr[e] * sc;
-            }
-        }
+    for (int e = 0; e < E; ++e) {
+        const long long k = i0 + e * span;
+        if (k < n) vj1[k] = wr[e] * sc;
     }
 }
 
@@ -1155,7 +1185,7 @@ static int coop_grid(hfh_ctx *c, int n) {
         per_cu < 1)
         return 0;
     const int G = std::max(c->num_cu, 1);
-    if (G > kCoopBlock || static_cast<long long>(G) * kCoopBlock * E < n) return 0;
+    if (kCoopSums * ((G + 63) / 64 * 64) > kCoopBlock || static_cast<long long>(G) * kCoopBlock * E < n) return 0;
     return G;
 }
 
@@ -1237,12 +1267,12 @@ static int gmres_impl(const hfh_csr *A, hfh_prec *P, int size_basis, int flexibl
             }
         }
     (void)hipGetLastError();
-    const int nstep = m1 + 1;   // steps of a column: j + 2 <= m + 1
+    const int nstep = (m1 + 1) / 2 + 1;   // sums of a column: the pairs of j + 1 <= m vectors, the norm
     unsigned long long *slots = nullptr;
     int *cfail = nullptr;
     int cseq = 0;
     if (cg > 0) {
-        const long long ns = 2LL * nstep * cg;
+        const long long ns = 2LL * nstep * kCoopSums * cg;
         if ((rc = w.alloc(reinterpret_cast<void **>(&slots), sizeof(unsigned long long) * ns)) ||
             (rc = w.alloc(reinterpret_cast<void **>(&cfail), sizeof(int))))
             return rc;
