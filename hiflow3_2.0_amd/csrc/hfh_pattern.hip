@@ -89,13 +89,13 @@ struct Lists {
 // neighbours by lane shifts and scalar loads 23.4 us; this form 22.0 us
 // (general layout, k_spmv_sellx: 99.0 us).
 // TRI: every group has three pairs; EXACT: there are U groups, one pass.
-// Slices whose window leaves x (the first and last ones) clamp a load per
-// pair.  Workgroups are dealt so that an XCD takes consecutive rows: nothing
+// Slices whose window leaves x (r0 + omin < 0, or r0 past `last`, the last first
+// row whose 64 rows' largest columns exist) clamp a load per pair.  Workgroups are dealt so that an XCD takes consecutive rows: nothing
 // but x is read more than once, and its window of a few grid planes stays in
 // the XCD's L2.
 template <typename T, bool ADD, bool DOT, int U, bool TRI, bool EXACT>
 __global__ __launch_bounds__(kBlock) void k_spmv_pattern(Lists<T> L, int nrow, int ncol, int nslice, int npair, int ngroup, int omin,
-                                                         int omax, const int *__restrict__ offs,
+                                                         int last, const int *__restrict__ offs,
                                                          const unsigned *__restrict__ set,
                                                          const int *__restrict__ partial, const T *__restrict__ x,
                                                          T *__restrict__ y, const T *__restrict__ w, double *part,
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_pattern(Lists<T> L, int nrow, i
         unsigned m = ~0u;
         if (cut) m = r < nrow ? set[r] : 0;
         T acc = 0;
-        if (r0 + omin >= 0 && r0 + 63 + omax < ncol) {
+        if (r0 + omin >= 0 && r0 <= last) {
             const T *xs = x + r0;
             auto add = [&](int k, T xk) {
                 const T t = add_rn(acc, mul_rn(L.val[k], xk));
@@ -158,7 +158,8 @@ __global__ __launch_bounds__(kBlock) void k_spmv_pattern(Lists<T> L, int nrow, i
             }
         } else {
             for (int k = 0; k < npair; ++k) {
-                const T xv = x[min(max(r + offs[k], 0), ncol - 1)];
+                const long long at = static_cast<long long>(r) + offs[k];
+                const T xv = x[min(max(at, 0LL), static_cast<long long>(ncol) - 1)];
                 const T t = add_rn(acc, mul_rn(L.val[k], xv));
                 acc = (m >> k) & 1u ? t : acc;
             }
@@ -301,8 +302,9 @@ template <typename T, bool ADD, bool DOT, int U, bool TRI, bool EXACT>
 void launch_u(const hfh_csr *A, const T *x, T *y, const T *w, double *part, const int *done) {
     Lists<T> L;
     std::memcpy(&L, A->pt_lists.data(), sizeof(L));
+    const long long last = std::min(static_cast<long long>(A->ncol) - 64 - A->pt_omax, 0x7fffffffLL);
     hipLaunchKernelGGL((k_spmv_pattern<T, ADD, DOT, U, TRI, EXACT>), dim3(A->nwg), dim3(kBlock), 0, A->ctx->stream, L,
-                       A->nrow, A->ncol, A->nslice, A->pt_pairs, A->pt_ngroups, A->pt_omin, A->pt_omax, A->pt_offs,
+                       A->nrow, A->ncol, A->nslice, A->pt_pairs, A->pt_ngroups, A->pt_omin, static_cast<int>(std::max(last, -1LL)), A->pt_offs,
                        A->pt_set, A->pt_partial, x, y, w, part, done);
 }
 
