@@ -20,8 +20,11 @@
 // and the sums over four rows of slots.  A workgroup returns its own entries
 // of a buffer to the sentinel when a later sum shows that everybody has read
 // them, and publishes its next A sum only when those stores have completed,
-// so nobody can poll the buffer again before.  Every wait is bounded; one
-// that gives up raises the failure word and the solve reports an error.
+// so nobody can poll the buffer again before.  Every wait is bounded: where
+// other work holds compute units for longer than that, so that some of the
+// workgroups cannot start, the launch ends with the failure word raised, the
+// initial guess (kept beside the solve) is put back and the launched form
+// solves the system.
 //
 // The step's arithmetic is the launched form's (cg.cc:163-248): row sums in
 // stored order with separate products and sums, FP64 sums over the rows in a
@@ -44,7 +47,7 @@ constexpr int kResBlock = 512;      // threads of a workgroup (one per CU)
 constexpr int kResWaves = kResBlock / 64;
 constexpr int kResRows = 4;         // slot rows of the sums
 constexpr int kCopies = 16;         // copies of each workgroup's sums
-constexpr int kResSpins = 1 << 16;
+constexpr int kResPolls = 1 << 16;   // of one wait: some tens of ms
 constexpr int kPre = 4;             // far z per thread received while the B sum is under way
 constexpr int kMaxGroups = 256;
 constexpr unsigned long long kResSentinel = 0x7FF4DEAD5EEDBEEFull;   // exponent all ones, quiet bit clear
@@ -68,12 +71,14 @@ __device__ __forceinline__ void far_store(U *p, U v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// polls p until it holds something else than the sentinel
+// polls p until it holds something else than the sentinel; a thread that has
+// given up once waits no more
 template <typename U>
-__device__ __forceinline__ U far_wait(const U *p, U u, U sentinel, int *s_fail) {
-    for (int spins = 0; u == sentinel; u = far_load(p))
-        if (++spins >= kResSpins) {
+__device__ __forceinline__ U far_wait(const U *p, U u, U sentinel, int &polls, int *s_fail) {
+    for (int k = 0; u == sentinel; u = far_load(p))
+        if (++k >= polls) {
             *s_fail = 1;
+            polls = 1;
             break;
         }
     return u;
@@ -97,6 +102,7 @@ struct ResidentArgs {
     double *out;              // pinned: iterations, state, residual, first residual, failure
     double atol, rtol, dtol;
     int maxits;
+    int polls;                // of one wait
 };
 
 // Sums of NQ values over the grid, the same bits in every thread: wave
@@ -107,8 +113,8 @@ struct ResidentArgs {
 // with 16 copies; 256: 2.9 and 2.3).  seq counts the sums; `between` runs
 // after the workgroup's sums are out.
 template <int NQ, typename F>
-__device__ __forceinline__ void grid_sum(double (&v)[NQ], int seq, unsigned long long *slots, double *sh, int *s_fail,
-                                         F between) {
+__device__ __forceinline__ void grid_sum(double (&v)[NQ], int seq, unsigned long long *slots, double *sh, int &polls,
+                                         int *s_fail, F between) {
     const int G = gridDim.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     double *s1 = sh + (seq & 1) * 4 * kResWaves, *s2 = s1 + 2 * kResWaves;
     static_assert(kResWaves == 8, "the sum of the waves");
@@ -140,7 +146,7 @@ __device__ __forceinline__ void grid_sum(double (&v)[NQ], int seq, unsigned long
         for (int q = 0; q < NQ; ++q) u[q] = tid < G ? far_load(mine + q * G + tid) : 0;
 #pragma unroll
         for (int q = 0; q < NQ; ++q) {
-            if (tid < G) u[q] = far_wait(mine + q * G + tid, u[q], kResSentinel, s_fail);
+            if (tid < G) u[q] = far_wait(mine + q * G + tid, u[q], kResSentinel, polls, s_fail);
             const double t = wave_sum_dpp(__builtin_bit_cast(double, u[q]));
             if (lane == 0) s2[q * kResWaves + w] = t;
         }
@@ -218,6 +224,7 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
     int seq = 1, it = 0, state = HFH_ITERATE;
     T beta = T(1);
     double res = 0, res0 = 0;
+    int polls = a.polls;
     bool failed = false;
     U zf[kPre];
     for (;;) {
@@ -233,7 +240,7 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
                 s[1] += static_cast<double>(r[e]) * static_cast<double>(z[e]);
             }
         }
-        grid_sum<2>(s, seq++, a.slots, sh, &s_fail, [&]() {
+        grid_sum<2>(s, seq++, a.slots, sh, polls, &s_fail, [&]() {
 #pragma unroll
             for (int q = 0; q < kPre; ++q) {
                 const int h = tid + q * kResBlock;
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
 #pragma unroll
             for (int q = 0; q < kPre; ++q) {
                 const int h = tid + q * kResBlock;
-                if (h < nfar) zf[q] = far_wait(reinterpret_cast<const U *>(zb) + w0 + far_pos(h), zf[q], kS, &s_far);
+                if (h < nfar) zf[q] = far_wait(reinterpret_cast<const U *>(zb) + w0 + far_pos(h), zf[q], kS, polls, &s_far);
             }
         });
         const T rrT = static_cast<T>(s[0]);
@@ -281,7 +288,7 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
                 const int h = h0 + q * kResBlock;
                 if (h < nfar) {
                     const int pos = far_pos(h);
-                    turn(pos, __builtin_bit_cast(T, far_wait(reinterpret_cast<const U *>(zb) + w0 + pos, u[q], kS, &s_far)));
+                    turn(pos, __builtin_bit_cast(T, far_wait(reinterpret_cast<const U *>(zb) + w0 + pos, u[q], kS, polls, &s_far)));
                 }
             }
         }
@@ -296,7 +303,7 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
         // this thread's returns to the sentinel have completed before its
         // workgroup's sum is published (the barrier in grid_sum)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        grid_sum<1>(t, seq++, a.slots, sh, &s_fail, []() {});
+        grid_sum<1>(t, seq++, a.slots, sh, polls, &s_fail, []() {});
         // everybody has formed its p of this step: the z of the last one is read
         if (G > 1) {
             U *const zo = reinterpret_cast<U *>(a.z[(it - 1) & 1]);
@@ -330,12 +337,15 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
     }
 }
 
-template <typename U>
-__global__ __launch_bounds__(kBlock) void k_resident_fill(int n, U *z0, U *z1, U v, int ns, unsigned long long *slots) {
+// Everything that is polled to the sentinel, and the initial guess kept.
+template <typename T, typename U>
+__global__ __launch_bounds__(kBlock) void k_resident_fill(int n, U *z0, U *z1, U v, int ns, unsigned long long *slots,
+                                                          const T *x, T *keep) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i < n) {
         z0[i] = v;
         z1[i] = v;
+        keep[i] = x[i];
     }
     if (i < ns) slots[i] = kResSentinel;
 }
@@ -359,7 +369,7 @@ static int resident_rows(const hfh_ctx *c, int n, int L) {
 }
 
 template <typename T, int L, int E>
-static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, bool &ran) {
+static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, T *keep, bool &ran) {
     hfh_ctx *c = A->ctx;
     const int R = kResBlock * E, G = (a.n + R - 1) / R;
     const size_t shm = sizeof(T) * (static_cast<size_t>(std::min(R + a.lo + a.hi, a.n)) + 1);
@@ -372,8 +382,9 @@ static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, bool &ran) {
     if (G > 1) {
         const int ns = kResRows * kCopies * 2 * G, m = std::max(a.n, ns);
         typedef typename Flag<T>::U U;
-        hipLaunchKernelGGL(k_resident_fill<U>, dim3((m + kBlock - 1) / kBlock), dim3(kBlock), 0, s, a.n,
-                           reinterpret_cast<U *>(a.z[0]), reinterpret_cast<U *>(a.z[1]), Flag<T>::sentinel, ns, a.slots);
+        hipLaunchKernelGGL((k_resident_fill<T, U>), dim3((m + kBlock - 1) / kBlock), dim3(kBlock), 0, s, a.n,
+                           reinterpret_cast<U *>(a.z[0]), reinterpret_cast<U *>(a.z[1]), Flag<T>::sentinel, ns, a.slots,
+                           (const T *)a.x, keep);
         if (int rc = launch_check("k_resident_fill")) return rc;
         void *args[] = {&a};
         // cooperative: all workgroups are resident together
@@ -390,8 +401,8 @@ static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, bool &ran) {
 }
 
 template <typename T>
-int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1, void *slots, double *hist,
-                const hfh_control &ctl, hfh_solve_info *info, bool *ran) {
+int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1, void *slots, T *keep,
+                double *hist, const hfh_control &ctl, hfh_solve_info *info, bool *ran) {
     *ran = false;
     hfh_ctx *c = A->ctx;
     const int n = A->nrow, L = A->shape_len;
@@ -402,13 +413,13 @@ int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1,
     if (window * static_cast<long long>(sizeof(T)) > kResidentLds || window >= 65536) return HFH_OK;
     ResidentArgs<T> a{n, A->shape_lo, A->shape_hi, A->row, A->col, static_cast<const T *>(A->val), b, invd, x, {z0, z1},
                       reinterpret_cast<unsigned long long *>(slots), hist, c->host_res, ctl.atol, ctl.rtol, ctl.dtol,
-                      ctl.maxits};
+                      ctl.maxits, c->wait_polls > 0 ? c->wait_polls : kResPolls};
     c->host_res[4] = 0;
     int rc;
 #define HFH_RES(LL)                                                         \
-    (E == 1 ? resident_launch<T, LL, 1>(A, a, *ran)                         \
-            : E == 2 ? resident_launch<T, LL, 2>(A, a, *ran)                \
-                     : resident_launch<T, LL, (LL <= 9 ? 4 : 2)>(A, a, *ran))
+    (E == 1 ? resident_launch<T, LL, 1>(A, a, keep, *ran)                         \
+            : E == 2 ? resident_launch<T, LL, 2>(A, a, keep, *ran)                \
+                     : resident_launch<T, LL, (LL <= 9 ? 4 : 2)>(A, a, keep, *ran))
     if (L <= 5) rc = HFH_RES(5);
     else if (L <= 7) rc = HFH_RES(7);
     else if (L <= 9) rc = HFH_RES(9);
@@ -417,7 +428,13 @@ int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1,
 #undef HFH_RES
     if (rc || !*ran) return rc;
     HFH_HIP(hipStreamSynchronize(c->stream));
-    HFH_CHECK(c->host_res[4] == 0, HFH_ERR_HIP, "CG: a workgroup gave up waiting for another one's values");
+    if (c->host_res[4] != 0) {   // x may hold some workgroups' rows of the solution
+        ++c->cg_gave_up;
+        *ran = false;
+        HFH_HIP(hipMemcpyAsync(x, keep, sizeof(T) * static_cast<size_t>(n), hipMemcpyDeviceToDevice, c->stream));
+        return HFH_OK;
+    }
+    ++c->cg_resident;
     info->iters = static_cast<int>(c->host_res[0]);
     info->state = static_cast<int>(c->host_res[1]);
     info->res = c->host_res[2];
@@ -426,8 +443,8 @@ int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1,
 }
 
 template int cg_resident<double>(const hfh_csr *, const double *, const double *, double *, double *, double *, void *,
-                                 double *, const hfh_control &, hfh_solve_info *, bool *);
+                                 double *, double *, const hfh_control &, hfh_solve_info *, bool *);
 template int cg_resident<float>(const hfh_csr *, const float *, const float *, float *, float *, float *, void *,
-                                double *, const hfh_control &, hfh_solve_info *, bool *);
+                                float *, double *, const hfh_control &, hfh_solve_info *, bool *);
 
 }  // namespace hfh

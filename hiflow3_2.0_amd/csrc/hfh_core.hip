@@ -493,6 +493,19 @@ extern "C" int hfh_ctx_timing_reset(hfh_ctx *c) {
     return HFH_OK;
 }
 
+extern "C" int hfh_ctx_set_wait_polls(hfh_ctx *c, int polls) {
+    HFH_CHECK(c && polls >= 0, HFH_ERR_INVALID, "hfh_ctx_set_wait_polls: bad argument");
+    c->wait_polls = polls;
+    return HFH_OK;
+}
+
+extern "C" int hfh_ctx_cg_launches(const hfh_ctx *c, long long *one_launch, long long *gave_up) {
+    HFH_CHECK(c && one_launch && gave_up, HFH_ERR_INVALID, "hfh_ctx_cg_launches: null argument");
+    *one_launch = c->cg_resident;
+    *gave_up = c->cg_gave_up;
+    return HFH_OK;
+}
+
 // ---------------------------------------------------------------- vectors
 
 extern "C" int hfh_vec_create(hfh_ctx *ctx, int n, int dtype, hfh_vec **out) {

@@ -64,6 +64,8 @@ struct hfh_ctx {
     int live = 0;                     // vectors, matrices and preconditioners created on the context
     // device address of this device's static scratch array (hfh_krylov.hip)
     void *scratch = nullptr;
+    int wait_polls = 0;               // hfh_ctx_set_wait_polls (0: each kernel's own)
+    long long cg_resident = 0, cg_gave_up = 0;   // one-launch CG solves, those that fell back
     // work space of the last Jacobi solve, for the next one (hfh_jacobi.hip)
     std::atomic<hfh::JacobiSpace *> jacobi{nullptr};
 };
@@ -330,13 +332,14 @@ int mcsgs_rz_slots(const hfh_prec *P);
 int prec_sync(hfh_prec *P);
 
 // CG of a small enough system in one launch (hfh_cgres.hip): x is the initial
-// guess and the result; z0, z1 and slots (n elements each) are work space.
-// *ran false: the system does not qualify and nothing was done.
+// guess and the result; z0, z1, slots and keep (n elements each) are work
+// space.  *ran false: the system does not qualify, or a wait gave up; x is the
+// initial guess as before.
 constexpr int kResidentRows = 4 * 512 * 256;
 constexpr long long kResidentLds = 158 * 1024;
 template <typename T>
-int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1, void *slots, double *hist,
-                const hfh_control &ctl, hfh_solve_info *info, bool *ran);
+int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1, void *slots, T *keep,
+                double *hist, const hfh_control &ctl, hfh_solve_info *info, bool *ran);
 
 // SGS / ILU0 sweeps by pencils (hfh_pencil.hip).  pencil_build leaves P->pen
 // empty where the pattern is not a full 5- / 7-point stencil of the grid

@@ -74,6 +74,8 @@ HIP_API = {
     "hfh_ctx_set_timing": (_i, [_vp, _i]),
     "hfh_ctx_timing": (_i, [_vp, _i, _P(_ll), _P(_d)]),
     "hfh_ctx_timing_reset": (_i, [_vp]),
+    "hfh_ctx_set_wait_polls": (_i, [_vp, _i]),
+    "hfh_ctx_cg_launches": (_i, [_vp, _P(_ll), _P(_ll)]),
     "hfh_vec_create": (_i, [_vp, _i, _i, _P(_vp)]),
     "hfh_vec_destroy": (_i, [_vp]),
     "hfh_vec_size": (_i, [_vp, _P(_i)]),
@@ -291,6 +293,16 @@ class Context:
 
     def timing_reset(self):
         _ck(hip().hfh_ctx_timing_reset(self.h))
+
+    def set_wait_polls(self, polls):
+        """Polls after which a one-launch kernel's wait gives up (0: its own bound)."""
+        _ck(hip().hfh_ctx_set_wait_polls(self.h, polls))
+
+    def cg_launches(self):
+        """(CG solves that ran as one launch, those that gave up and fell back)."""
+        a, b = C.c_longlong(), C.c_longlong()
+        _ck(hip().hfh_ctx_cg_launches(self.h, C.byref(a), C.byref(b)))
+        return a.value, b.value
 
 
 class Vector:

@@ -63,6 +63,14 @@ int hfh_ctx_info(hfh_ctx *ctx, int *num_cu, long long *hbm_bytes, char *name, in
 int hfh_ctx_set_timing(hfh_ctx *ctx, int on);
 int hfh_ctx_timing(hfh_ctx *ctx, int kclass, long long *launches, double *total_ms);
 int hfh_ctx_timing_reset(hfh_ctx *ctx);
+/* polls after which a wait between the workgroups of a one-launch CG gives up
+ * and the launched form takes over (no reference counterpart): 0, the default,
+ * is the kernel's own bound of some tens of ms; 1 gives up at the first value
+ * that is not there yet */
+int hfh_ctx_set_wait_polls(hfh_ctx *ctx, int polls);
+/* CG solves of the context that ran as one launch, and those whose launch
+ * gave up waiting and that the launched form then solved */
+int hfh_ctx_cg_launches(const hfh_ctx *ctx, long long *one_launch, long long *gave_up);
 
 /* ---- vectors: lVector<T> (lmp/lvector.h:39-336) ---- */
 /* lVector::Init (lvector.h:199) + CloneWithoutContent (lvector.cc:52-64): zero filled */
@@ -341,8 +349,9 @@ typedef struct {
  * automatic SpMV layout, at most 28 entries per row and a system that fits on
  * the chip (up to 524,288 rows of up to 9 entries, 262,144 otherwise; columns
  * within about 10,000 rows in FP64), the whole solve is one cooperative
- * launch (HFH_ERR_HIP if one of its bounded waits gave up).  Returns HFH_OK on convergence,
- * HFH_ERR_NOT_CONVERGED on maxits/divergence (info is filled either way).
+ * launch.  Where one of its bounded waits gives up (other work kept part of
+ * its workgroups from starting) the solve begins again from the initial guess
+ * in the launched form.  Returns HFH_OK on convergence, HFH_ERR_NOT_CONVERGED on maxits/divergence (info is filled either way).
  * An empty system (n = 0) returns at once: 0 iterations, residual 0,
  * state HFH_SUCCESS_ABS (the same holds for GMRES and defect correction).
  * hist (optional, host, maxits+1 doubles) receives the residual history. */
