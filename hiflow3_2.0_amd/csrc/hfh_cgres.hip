@@ -33,7 +33,9 @@
 // Measured per step (Jacobi, FP64; launched -> resident): 1,517 rows (2D FV,
 // one workgroup) 13.8 -> 2.7 us, 8,000 rows (3D Q1) 22.6 -> 6.6, 65,025 rows
 // (2D Q1) 14.8 -> 5.7, 125,000 rows (3D Q1) 22.8 -> 10.0, 250,047 rows (3D FV)
-// 19.3 -> 11.3, 490,000 rows (2D Q1) 30.4 -> 8.0.  What remains is the two
+// 19.3 -> 11.3, 490,000 rows (2D Q1) 30.4 -> 8.0.  The largest form (3D Q1,
+// two rows of 27 entries per thread) takes 10.8 us at 175,616 rows and 13.0 at
+// 250,047; with its codes unpacked once and 86 registers spilled 12.3 and 16.8.  What remains is the two
 // sums (1.8 us each on 128 workgroups) and the far z.
 #include "hfh_internal.h"
 
@@ -181,6 +183,12 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
     const int w0 = max(0, r0 - a.lo), w1 = r1 > a.n - a.hi ? a.n : r1 + a.hi;
     const int wlen = w1 - w0, own0 = r0 - w0, nown = r1 - r0, nfar = wlen - nown;
     auto far_pos = [&](int h) { return h < own0 ? h : h + nown; };
+    // The largest form's values and codes leave few registers, and its first
+    // launch must not make the runtime reserve scratch.  It unpacks its codes
+    // anew in every step (`step` hides that they never change; the compiler
+    // kept all unpacked codes too and spilled 86 registers) and reads the rows
+    // once more for the first residual.
+    constexpr bool kFew = sizeof(T) * L * E > 256;
     T v[E][L], xr[E], r[E], z[E], d[E], Ap[E];
     unsigned code[E][(L + 1) / 2];
     bool in[E];
@@ -202,18 +210,33 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
         }
     }
     __syncthreads();
-    auto spmv = [&]() {
+    auto spmv = [&](int step) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             T s = T(0);
 #pragma unroll
-            for (int k = 0; k < L; ++k)
-                s = add_rn(s, mul_rn(v[e][k], pw[(k & 1) ? code[e][k >> 1] >> 16 : code[e][k >> 1] & 0xffffu]));
+            for (int k = 0; k < L; k += 2) {
+                unsigned c = code[e][k >> 1];
+                if (kFew) asm("" : "+v"(c) : "v"(step));
+                s = add_rn(s, mul_rn(v[e][k], pw[c & 0xffffu]));
+                if (k + 1 < L) s = add_rn(s, mul_rn(v[e][k + 1], pw[c >> 16]));
+            }
             Ap[e] = s;
         }
     };
     // step 0: r = b - A x
-    spmv();
+    if (kFew) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int i = r0 + e * kResBlock + tid, j0 = in[e] ? a.row[i] : 0, j1 = in[e] ? a.row[i + 1] : 0;
+            T s = T(0);
+#pragma unroll 4
+            for (int j = j0; j < j1; ++j) s = add_rn(s, mul_rn(a.val[j], pw[a.col[j] - w0]));
+            Ap[e] = s;
+        }
+    } else {
+        spmv(0);
+    }
     double s[2] = {0, 0};
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -295,7 +318,7 @@ __global__ __launch_bounds__(kResBlock) void k_cg_resident(ResidentArgs<T> a) {
         __syncthreads();
         // ---- A: Ap, the sum of p.Ap, alpha
         ++it;
-        spmv();
+        spmv(it);
         double t[1] = {0};
 #pragma unroll
         for (int e = 0; e < E; ++e)
@@ -369,7 +392,7 @@ static int resident_rows(const hfh_ctx *c, int n, int L) {
 }
 
 template <typename T, int L, int E>
-static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, T *keep, bool &ran) {
+static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, T *keep, bool noalloc, bool &ran) {
     hfh_ctx *c = A->ctx;
     const int R = kResBlock * E, G = (a.n + R - 1) / R;
     const size_t shm = sizeof(T) * (static_cast<size_t>(std::min(R + a.lo + a.hi, a.n)) + 1);
@@ -387,8 +410,14 @@ static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, T *keep, bool &
                            (const T *)a.x, keep);
         if (int rc = launch_check("k_resident_fill")) return rc;
         void *args[] = {&a};
-        // cooperative: all workgroups are resident together
-        if (hipLaunchCooperativeKernel(f, dim3(G), dim3(kResBlock), args, static_cast<unsigned>(shm), s) != hipSuccess) {
+        // Cooperative launches of one process run one after the other, so two
+        // solves never hold half of the compute units each.  The first one
+        // makes the runtime allocate a queue (8 MB); where nothing may be
+        // allocated a plain launch has the bounded waits to rely on.
+        if (noalloc) {
+            hipLaunchKernelGGL((k_cg_resident<T, L, E>), dim3(G), dim3(kResBlock), shm, s, a);
+            if (int rc = launch_check("k_cg_resident")) return rc;
+        } else if (hipLaunchCooperativeKernel(f, dim3(G), dim3(kResBlock), args, static_cast<unsigned>(shm), s) != hipSuccess) {
             (void)hipGetLastError();
             return HFH_OK;
         }
@@ -400,9 +429,15 @@ static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, T *keep, bool &
     return HFH_OK;
 }
 
+int resident_load() {
+    hipFuncAttributes attr;
+    HFH_HIP(hipFuncGetAttributes(&attr, reinterpret_cast<const void *>(k_cg_resident<double, 5, 1>)));
+    return HFH_OK;
+}
+
 template <typename T>
 int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1, void *slots, T *keep,
-                double *hist, const hfh_control &ctl, hfh_solve_info *info, bool *ran) {
+                double *hist, const hfh_control &ctl, bool noalloc, hfh_solve_info *info, bool *ran) {
     *ran = false;
     hfh_ctx *c = A->ctx;
     const int n = A->nrow, L = A->shape_len;
@@ -417,9 +452,9 @@ int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1,
     c->host_res[4] = 0;
     int rc;
 #define HFH_RES(LL)                                                         \
-    (E == 1 ? resident_launch<T, LL, 1>(A, a, keep, *ran)                         \
-            : E == 2 ? resident_launch<T, LL, 2>(A, a, keep, *ran)                \
-                     : resident_launch<T, LL, (LL <= 9 ? 4 : 2)>(A, a, keep, *ran))
+    (E == 1 ? resident_launch<T, LL, 1>(A, a, keep, noalloc, *ran)                         \
+            : E == 2 ? resident_launch<T, LL, 2>(A, a, keep, noalloc, *ran)                \
+                     : resident_launch<T, LL, (LL <= 9 ? 4 : 2)>(A, a, keep, noalloc, *ran))
     if (L <= 5) rc = HFH_RES(5);
     else if (L <= 7) rc = HFH_RES(7);
     else if (L <= 9) rc = HFH_RES(9);
@@ -443,8 +478,8 @@ int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1,
 }
 
 template int cg_resident<double>(const hfh_csr *, const double *, const double *, double *, double *, double *, void *,
-                                 double *, double *, const hfh_control &, hfh_solve_info *, bool *);
+                                 double *, double *, const hfh_control &, bool, hfh_solve_info *, bool *);
 template int cg_resident<float>(const hfh_csr *, const float *, const float *, float *, float *, float *, void *,
-                                float *, double *, const hfh_control &, hfh_solve_info *, bool *);
+                                float *, double *, const hfh_control &, bool, hfh_solve_info *, bool *);
 
 }  // namespace hfh

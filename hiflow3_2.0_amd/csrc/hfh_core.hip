@@ -427,8 +427,8 @@ extern "C" int hfh_ctx_create(int device, hfh_ctx **out) {
     HFH_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->host_res), sizeof(double) * 256));
     HFH_HIP(hipEventCreate(&c->ev0));
     HFH_HIP(hipEventCreate(&c->ev1));
-    // the allocation-free CG's static array on this device (current now)
-    if ((rc = static_scratch(device, &c->scratch))) {
+    // the allocation-free CG's static array on this device (current now) and its code
+    if ((rc = static_scratch(device, &c->scratch)) || (rc = resident_load())) {
         (void)hipStreamDestroy(c->stream);
         (void)hipFree(c->red);
         (void)hipHostFree(c->host_res);

@@ -331,15 +331,19 @@ int mcsgs_rz_slots(const hfh_prec *P);
 // matrix's values changed); a no-op while the stream is being captured.
 int prec_sync(hfh_prec *P);
 
+// Loads the one-launch CG's code (2 MB of device memory), so that the first
+// allocation-free solve does not.
+int resident_load();
 // CG of a small enough system in one launch (hfh_cgres.hip): x is the initial
 // guess and the result; z0, z1, slots and keep (n elements each) are work
 // space.  *ran false: the system does not qualify, or a wait gave up; x is the
-// initial guess as before.
+// initial guess as before.  noalloc: nothing is allocated, by the runtime
+// neither.
 constexpr int kResidentRows = 4 * 512 * 256;
 constexpr long long kResidentLds = 158 * 1024;
 template <typename T>
 int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1, void *slots, T *keep,
-                double *hist, const hfh_control &ctl, hfh_solve_info *info, bool *ran);
+                double *hist, const hfh_control &ctl, bool noalloc, hfh_solve_info *info, bool *ran);
 
 // SGS / ILU0 sweeps by pencils (hfh_pencil.hip).  pencil_build leaves P->pen
 // empty where the pattern is not a full 5- / 7-point stencil of the grid

@@ -711,7 +711,7 @@ struct PcgWork {
         if (R.mode != 2 && !keep_direction) {
             hfh_solve_info ri{};
             bool ran = false;
-            rc = cg_resident<T>(A, R.invd, b, x, R.z, R.Ap, R.p, R.r, hist, ctl, &ri, &ran);
+            rc = cg_resident<T>(A, R.invd, b, x, R.z, R.Ap, R.p, R.r, hist, ctl, noalloc, &ri, &ran);
             if (rc) return rc;
             if (ran) return finish_resident(ri, info, hhist, noalloc, e0, e1, t0);
         }

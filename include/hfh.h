@@ -367,8 +367,9 @@ int hfh_pcg_solve(const hfh_csr *A, hfh_prec *P, const hfh_vec *b, hfh_vec *x,
  * maxits + 2 doubles with hist), so FP64 systems up to about 2.09 M rows,
  * FP32 up to about 4.19 M; larger solves return HFH_ERR_INVALID.  P must be
  * NULL, HFH_PREC_NONE or Jacobi (else HFH_ERR_UNSUPPORTED).  Same iterates,
- * stopping test and results as hfh_pcg_solve; the loop runs as direct
- * launches (no graph) and info->time_ms is host wall time.  Every call on
+ * stopping test and results as hfh_pcg_solve, in the same form: one launch
+ * (plain instead of cooperative, whose queue the runtime would allocate), or
+ * the loop as direct launches (no graph).  info->time_ms is host wall time.  Every call on
  * one device shares the array: calls that overlap on one device race. */
 int hfh_pcg_solve_noalloc(const hfh_csr *A, hfh_prec *P, const hfh_vec *b, hfh_vec *x,
                           const hfh_control *ctl, hfh_solve_info *info, double *hist);
