@@ -149,25 +149,31 @@ __global__ __launch_bounds__(kBlock) void k_dot(int n, long long nv, const T *__
 // store over a signalling-NaN sentinel, which sums never yield, and workgroup
 // 0 polls all of them, returns them to the sentinel and adds them in
 // k_fin_store's order.  Nobody waits for workgroup 0, so it needs no
-// co-residency; its wait is bounded.  Above that a finisher launch costs less
-// than one workgroup's polls.
+// co-residency; its wait is bounded, and where it gives up (other work kept the
+// later workgroups from starting for seconds) the host empties the slots and
+// takes the finisher.  Above that a finisher launch costs less than one
+// workgroup's polls.
 constexpr int kDotOne = 1024;
 constexpr unsigned long long kDotSentinel = 0x7FF4DEAD5EEDBEEFull;   // exponent all ones, quiet bit clear
-constexpr int kDotSpins = 1 << 22;
+constexpr unsigned long long kDotGaveUp = kDotSentinel ^ 1;           // the host's word instead of a sum
+constexpr int kDotPolls = 1 << 22;
 static_assert(kDotOne == kFinBlock && kDotOne == 4 * kBlock, "workgroup 0 stands in for one pass of the finisher");
 
 __device__ __forceinline__ void host_store(double *p, double v) {
-    // a sum is never the sentinel; a NaN that carries its bits would be
+    // a sum is never one of the marks; a NaN that carries its bits would be
     unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-    if (u == kDotSentinel) u |= 1ull << 51;
+    if (u == kDotSentinel || u == kDotGaveUp) u |= 1ull << 51;
     __hip_atomic_store(reinterpret_cast<unsigned long long *>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_dot_host(int n, long long nv, const T *__restrict__ x,
-                                                     const T *__restrict__ y, unsigned long long *slots, double *dst) {
+                                                     const T *__restrict__ y, unsigned long long *slots, int polls,
+                                                     double *dst) {
     __shared__ double sh[kFinBlock / 64], bc;
     __shared__ double got[kDotOne];
+    __shared__ int gave_up;
+    if (threadIdx.x == 0) gave_up = 0;
     const double v = dot_part<T, false>(n, nv, x, y, sh);
     const int nb = gridDim.x;
     if (threadIdx.x == 0) {
@@ -178,15 +184,24 @@ __global__ __launch_bounds__(kBlock) void k_dot_host(int n, long long nv, const 
     if (blockIdx.x != 0) return;
     for (int b = threadIdx.x; b < nb; b += kBlock) {
         unsigned long long u = kDotSentinel;
-        for (int spin = 0; u == kDotSentinel && spin < kDotSpins; ++spin)
+        for (int k = 0; u == kDotSentinel && k < polls; ++k)
             u = __hip_atomic_load(slots + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (u == kDotSentinel) gave_up = 1;
         __hip_atomic_store(slots + b, kDotSentinel, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        got[b] = __builtin_bit_cast(double, u);   // given up: the sentinel's NaN
+        got[b] = __builtin_bit_cast(double, u);
     }
     __syncthreads();
+    if (gave_up) {
+        if (threadIdx.x == 0)
+            __hip_atomic_store(reinterpret_cast<unsigned long long *>(dst), kDotGaveUp, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
+    }
     const double s = fin_sum_all(got, nb, sh, &bc);
     if (threadIdx.x == 0) host_store(dst, s);
 }
+
+__global__ __launch_bounds__(kDotOne) void k_dot_empty(unsigned long long *slots) { slots[threadIdx.x] = kDotSentinel; }
 
 // 16-byte vectors of both operands when both are aligned, else none.
 template <typename T>
@@ -239,26 +254,35 @@ static int dot_partials(hfh_ctx *ctx, int dtype, int n, const void *x, const voi
 // The dot of n > 0 elements, waited for by polling a word of pinned memory.
 static int dot_host(hfh_ctx *ctx, int dtype, int n, const void *x, const void *y, double *out) {
     volatile unsigned long long *word = reinterpret_cast<volatile unsigned long long *>(ctx->host_res + kHostDot);
-    *word = kDotSentinel;
     double *dst = ctx->host_res + kHostDot;
+    const int polls = ctx->wait_polls > 0 ? ctx->wait_polls : kDotPolls;
     int nb = red_blocks(n, kDotBlocks), rc;
-    if (nb <= kDotOne) {
-        if (dtype == HFH_F64)
-            hipLaunchKernelGGL(k_dot_host<double>, dim3(nb), dim3(kBlock), 0, ctx->stream, n, vec_count<double>(n, x, y),
-                               (const double *)x, (const double *)y, ctx->dot_slots, dst);
-        else
-            hipLaunchKernelGGL(k_dot_host<float>, dim3(nb), dim3(kBlock), 0, ctx->stream, n, vec_count<float>(n, x, y),
-                               (const float *)x, (const float *)y, ctx->dot_slots, dst);
-        rc = launch_check("k_dot_host");
-    } else if (!(rc = dot_partials(ctx, dtype, n, x, y, &nb))) {
-        hipLaunchKernelGGL(k_fin_host, dim3(1), dim3(kFinBlock), 0, ctx->stream, (const double *)ctx->red, nb, dst);
-        rc = launch_check("k_fin_host");
+    bool one = nb <= kDotOne;
+    for (;;) {
+        *word = kDotSentinel;
+        if (one) {
+            if (dtype == HFH_F64)
+                hipLaunchKernelGGL(k_dot_host<double>, dim3(nb), dim3(kBlock), 0, ctx->stream, n, vec_count<double>(n, x, y),
+                                   (const double *)x, (const double *)y, ctx->dot_slots, polls, dst);
+            else
+                hipLaunchKernelGGL(k_dot_host<float>, dim3(nb), dim3(kBlock), 0, ctx->stream, n, vec_count<float>(n, x, y),
+                                   (const float *)x, (const float *)y, ctx->dot_slots, polls, dst);
+            rc = launch_check("k_dot_host");
+        } else if (!(rc = dot_partials(ctx, dtype, n, x, y, &nb))) {
+            hipLaunchKernelGGL(k_fin_host, dim3(1), dim3(kFinBlock), 0, ctx->stream, (const double *)ctx->red, nb, dst);
+            rc = launch_check("k_fin_host");
+        }
+        if (rc) return rc;
+        // short waits by polling; past about a millisecond, and for any error of
+        // the queued work, the stream's own synchronisation
+        for (int spin = 0; spin < 1 << 15 && *word == kDotSentinel; ++spin) __builtin_ia32_pause();
+        if (*word == kDotSentinel) HFH_HIP(hipStreamSynchronize(ctx->stream));
+        if (*word != kDotGaveUp) break;
+        // the workgroups that came late have stored their partials after all
+        hipLaunchKernelGGL(k_dot_empty, dim3(1), dim3(kDotOne), 0, ctx->stream, ctx->dot_slots);
+        if ((rc = launch_check("k_dot_empty"))) return rc;
+        one = false;
     }
-    if (rc) return rc;
-    // short waits by polling; past about a millisecond, and for any error of
-    // the queued work, the stream's own synchronisation
-    for (int spin = 0; spin < 1 << 15 && *word == kDotSentinel; ++spin) __builtin_ia32_pause();
-    if (*word == kDotSentinel) HFH_HIP(hipStreamSynchronize(ctx->stream));
     HFH_CHECK(*word != kDotSentinel, HFH_ERR_HIP, "hfh_dot: the result did not arrive");
     std::atomic_thread_fence(std::memory_order_acquire);
     const unsigned long long u = *word;

@@ -63,10 +63,10 @@ int hfh_ctx_info(hfh_ctx *ctx, int *num_cu, long long *hbm_bytes, char *name, in
 int hfh_ctx_set_timing(hfh_ctx *ctx, int on);
 int hfh_ctx_timing(hfh_ctx *ctx, int kclass, long long *launches, double *total_ms);
 int hfh_ctx_timing_reset(hfh_ctx *ctx);
-/* polls after which a wait between the workgroups of a one-launch CG gives up
- * and the launched form takes over (no reference counterpart): 0, the default,
- * is the kernel's own bound of some tens of ms; 1 gives up at the first value
- * that is not there yet */
+/* polls after which a wait between the workgroups of a one-launch CG or dot
+ * gives up and the form of several launches takes over (no reference
+ * counterpart): 0, the default, is the kernel's own bound (CG some tens of ms,
+ * dot some seconds); 1 gives up at the first value that is not there yet */
 int hfh_ctx_set_wait_polls(hfh_ctx *ctx, int polls);
 /* CG solves of the context that ran as one launch, and those whose launch
  * gave up waiting and that the launched form then solved */

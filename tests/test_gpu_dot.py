@@ -33,3 +33,20 @@ def test_host_dot_special_values(pkg, ctx, n):
         got = pkg.Vector(ctx, x).dot(one)
         assert got == v if np.isinf(v) else np.isnan(got)
     assert one.dot(one) == n        # the next dot is not affected
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [513, 65025, 262144])
+def test_dot_that_gives_up_waiting(pkg, ctx, n, dtype):
+    """A one-launch dot that does not wait for its partials hands over to the
+    finisher: the same bits, and partials that came late reach no later dot."""
+    rng = np.random.default_rng(n)
+    vecs = [pkg.Vector(ctx, rng.uniform(-1, 1, n), dtype) for _ in range(6)]
+    want = [v.dot(vecs[0]) for v in vecs]
+    for rep in range(3):
+        ctx.set_wait_polls(1)
+        try:
+            assert [v.dot(vecs[0]) for v in vecs] == want
+        finally:
+            ctx.set_wait_polls(0)
+        assert [v.dot(vecs[0]) for v in vecs] == want
