@@ -43,6 +43,15 @@ int dev_alloc(void **p, size_t bytes) {
     return HFH_OK;
 }
 
+int copy_alloc(hfh_ctx *c, void **p, size_t bytes) {
+    *p = nullptr;
+    if (c->copy_limit > 0 && bytes > static_cast<unsigned long long>(c->copy_limit)) {
+        set_error("a copy of %zu bytes is above the context's limit", bytes);
+        return HFH_ERR_NOMEM;
+    }
+    return dev_alloc(p, bytes);
+}
+
 int launch_check(const char *what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, what);
@@ -527,6 +536,12 @@ extern "C" int hfh_ctx_cg_launches(const hfh_ctx *c, long long *one_launch, long
     HFH_CHECK(c && one_launch && gave_up, HFH_ERR_INVALID, "hfh_ctx_cg_launches: null argument");
     *one_launch = c->cg_resident;
     *gave_up = c->cg_gave_up;
+    return HFH_OK;
+}
+
+extern "C" int hfh_ctx_set_copy_limit(hfh_ctx *c, long long bytes) {
+    HFH_CHECK(c && bytes >= 0, HFH_ERR_INVALID, "hfh_ctx_set_copy_limit: bad argument");
+    c->copy_limit = bytes;
     return HFH_OK;
 }
 

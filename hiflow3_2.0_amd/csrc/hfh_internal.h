@@ -65,6 +65,7 @@ struct hfh_ctx {
     // device address of this device's static scratch array (hfh_krylov.hip)
     void *scratch = nullptr;
     int wait_polls = 0;               // hfh_ctx_set_wait_polls (0: each kernel's own)
+    long long copy_limit = 0;         // hfh_ctx_set_copy_limit (0: none)
     long long cg_resident = 0, cg_gave_up = 0;   // one-launch CG solves, those that fell back
     // work space of the last Jacobi solve, for the next one (hfh_jacobi.hip)
     std::atomic<hfh::JacobiSpace *> jacobi{nullptr};
@@ -264,6 +265,9 @@ inline int hip_fail(hipError_t e, const char *what) {
     } while (0)
 
 int dev_alloc(void **p, size_t bytes);
+// For copies of a matrix that only make it faster: HFH_ERR_NOMEM (also above
+// the context's limit) means that the caller does without.
+int copy_alloc(hfh_ctx *c, void **p, size_t bytes);
 int launch_check(const char *what);
 // False when the environment sets HFH_GRAPHS=0: the drivers and the serving
 // engine then launch every iteration directly instead of replaying a

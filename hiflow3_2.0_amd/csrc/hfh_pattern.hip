@@ -199,8 +199,8 @@ int fill(hfh_csr *A) {
                  at_fail = at_rows + sizeof(int) * np, at_part = at_fail + sizeof(int),
                  at_set = at_part + sizeof(int) * nsl, bytes = at_set + sizeof(unsigned) * static_cast<size_t>(n);
     if (!A->pt_block) {
-        const int rc = dev_alloc(&A->pt_block, bytes);
-        if (rc) return rc;
+        const int rc = copy_alloc(A->ctx, &A->pt_block, bytes);
+        if (rc) return rc == HFH_ERR_NOMEM ? HFH_OK : rc;   // the general layout serves
     }
     char *blk = static_cast<char *>(A->pt_block);
     T *d_vals = reinterpret_cast<T *>(blk + at_vals);

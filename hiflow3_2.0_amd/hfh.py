@@ -75,6 +75,7 @@ HIP_API = {
     "hfh_ctx_timing": (_i, [_vp, _i, _P(_ll), _P(_d)]),
     "hfh_ctx_timing_reset": (_i, [_vp]),
     "hfh_ctx_set_wait_polls": (_i, [_vp, _i]),
+    "hfh_ctx_set_copy_limit": (_i, [_vp, _ll]),
     "hfh_ctx_cg_launches": (_i, [_vp, _P(_ll), _P(_ll)]),
     "hfh_vec_create": (_i, [_vp, _i, _i, _P(_vp)]),
     "hfh_vec_destroy": (_i, [_vp]),
@@ -297,6 +298,10 @@ class Context:
     def set_wait_polls(self, polls):
         """Polls after which a one-launch kernel's wait gives up (0: its own bound)."""
         _ck(hip().hfh_ctx_set_wait_polls(self.h, polls))
+
+    def set_copy_limit(self, size):
+        """Bytes one optional copy of a matrix may take (0: no limit)."""
+        _ck(hip().hfh_ctx_set_copy_limit(self.h, size))
 
     def cg_launches(self):
         """(CG solves that ran as one launch, those that gave up and fell back)."""

@@ -131,3 +131,22 @@ def test_values_change(pkg, ctx):
     assert pkg.CsrMatrix.cast_of(A, np.float32).pattern_pairs() == 27
     A.swap_diag_front()      # the row order is no longer ascending
     assert A.pattern_pairs() == 0
+
+
+def test_no_room_for_the_list(pkg, ctx):
+    """Without memory for the list every call that would make it succeeds in
+    the general layout: upload, new values, another layout and back, a cast."""
+    shape = (12, 13, 70)
+    row, col, val = stencil(shape, *box(3))
+    ctx.set_copy_limit(1)
+    try:
+        A = compare(pkg, ctx, row, col, val, np.float64, 0)
+        A.upload_values(2 * val)
+        A.scale(0.5)
+        A.set_spmv(pkg.SPMV_SELL_PAIRS, 1)
+        A.set_spmv(pkg.SPMV_AUTO)
+        assert A.pattern_pairs() == 0 and pkg.CsrMatrix.cast_of(A, np.float32).pattern_pairs() == 0
+    finally:
+        ctx.set_copy_limit(0)
+    A.upload_values(val)
+    assert A.pattern_pairs() == 27
