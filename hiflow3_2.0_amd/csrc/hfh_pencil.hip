@@ -585,12 +585,14 @@ int pencil_build(hfh_prec *P, int nx, long long nxy) {
     // the skew's idle steps must not dominate the value copies
     const long long slots = 256LL * G.np * G.ng;
     if (slots > 4LL * n) return HFH_OK;
+    hfh_ctx *c = P->ctx;
     int rc;
-    if ((rc = dev_alloc(reinterpret_cast<void **>(&G.ctl), sizeof(int) * 96))) return rc;
+    // no memory for the pencils: the blocks take a part of it
     auto give_up = [&](int code) {
         pencil_free(G);
-        return code;
+        return code == HFH_ERR_NOMEM ? static_cast<int>(HFH_OK) : code;
     };
+    if ((rc = copy_alloc(c, reinterpret_cast<void **>(&G.ctl), sizeof(int) * 96))) return give_up(rc);
     int bad = 0;
     hipError_t e = hipMemsetAsync(G.ctl, 0, sizeof(int) * 96, s);
     if (e != hipSuccess) return give_up(hip_fail(e, "hipMemsetAsync"));
@@ -612,10 +614,10 @@ int pencil_build(hfh_prec *P, int nx, long long nxy) {
     const int nv = d3 ? 3 : 2, kf = nv + (P->kind == HFH_PREC_ILU0 ? 0 : 2), kb = nv + 2, H = d3 ? 16 : 1;
     const long long nbox = static_cast<long long>(G.np) * G.ng * 4 * H;
     const size_t ysize = static_cast<size_t>(es) * G.np * (4 * G.ng + 4) * 64;
-    if ((rc = dev_alloc(reinterpret_cast<void **>(&G.order), sizeof(int) * G.np)) ||
-        (rc = dev_alloc(&G.fval, static_cast<size_t>(es * slots * kf))) ||
-        (rc = dev_alloc(&G.bval, static_cast<size_t>(es * slots * kb))) || (rc = dev_alloc(&G.y, ysize)) ||
-        (rc = dev_alloc(&G.fbox, static_cast<size_t>(es * nbox))) || (rc = dev_alloc(&G.bbox, static_cast<size_t>(es * nbox))))
+    if ((rc = copy_alloc(c, reinterpret_cast<void **>(&G.order), sizeof(int) * G.np)) ||
+        (rc = copy_alloc(c, &G.fval, static_cast<size_t>(es * slots * kf))) ||
+        (rc = copy_alloc(c, &G.bval, static_cast<size_t>(es * slots * kb))) || (rc = copy_alloc(c, &G.y, ysize)) ||
+        (rc = copy_alloc(c, &G.fbox, static_cast<size_t>(es * nbox))) || (rc = copy_alloc(c, &G.bbox, static_cast<size_t>(es * nbox))))
         return give_up(rc);
     e = hipMemcpyAsync(G.order, order.data(), sizeof(int) * G.np, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemsetAsync(G.y, 0, ysize, s);

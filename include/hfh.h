@@ -69,8 +69,8 @@ int hfh_ctx_timing_reset(hfh_ctx *ctx);
  * dot some seconds); 1 gives up at the first value that is not there yet */
 int hfh_ctx_set_wait_polls(hfh_ctx *ctx, int polls);
 /* device bytes that one copy of a matrix may take where a slower form does
- * without it: the list of repeated pairs of an SpMV (no reference counterpart);
- * 0, the default, is no limit.  A copy that is above the limit, or that the
+ * without it: the list of repeated pairs of an SpMV, the pencils of a sweep (no
+ * reference counterpart); 0, the default, is no limit.  A copy that is above the limit, or that the
  * device has no memory for, is left out and the call succeeds. */
 int hfh_ctx_set_copy_limit(hfh_ctx *ctx, long long bytes);
 /* CG solves of the context that ran as one launch, and those whose launch

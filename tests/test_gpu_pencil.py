@@ -102,3 +102,23 @@ def test_other_patterns_keep_their_schedule(pkg, oracle, ctx, what):
     Y = pkg.Vector(ctx, n)
     M.apply(pkg.Vector(ctx, rhs), Y)
     assert np.array_equal(Y.numpy(), oracle.sgs(oracle.Csr(row, col, val), rhs))
+
+
+@pytest.mark.parametrize("shape", [(70, 66, 1), (18, 17, 16)])
+@pytest.mark.parametrize("limit", [1, 4096])
+def test_no_room_for_the_pencils(pkg, oracle, ctx, shape, limit):
+    """Without memory for the first or a later one of the pencils' copies the
+    preconditioner is created all the same and sweeps by blocks."""
+    row, col, val, rhs = system(pkg, shape)
+    A = pkg.CsrMatrix(ctx, row, col, val)
+    ctx.set_copy_limit(limit)
+    try:
+        M = pkg.Preconditioner.sgs(A, row, col)
+    finally:
+        ctx.set_copy_limit(0)
+    pencils = pkg.Preconditioner.sgs(A, row, col).sweep_blocks()
+    assert M.sweep_blocks()[0] > pencils[0] > 0
+    Y = pkg.Vector(ctx, len(rhs))
+    M.apply(pkg.Vector(ctx, rhs), Y)
+    M.sweep_status()
+    assert same(Y.numpy(), oracle.sgs(oracle.Csr(row, col, val), rhs))
