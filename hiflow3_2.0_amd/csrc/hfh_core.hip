@@ -457,7 +457,8 @@ extern "C" int hfh_ctx_create(int device, hfh_ctx **out) {
     c->dot_slots = reinterpret_cast<unsigned long long *>(c->red + kRedBlocks * 8 + 256);
     const std::vector<unsigned long long> empty(kDotOne, kDotSentinel);
     HFH_HIP(hipMemcpy(c->dot_slots, empty.data(), sizeof(unsigned long long) * kDotOne, hipMemcpyHostToDevice));
-    HFH_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->host_res), sizeof(double) * 256));
+    HFH_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->host_res), sizeof(double) * 256 + kReportBytes));
+    c->host_reports = c->host_res + 256;
     HFH_HIP(hipEventCreate(&c->ev0));
     HFH_HIP(hipEventCreate(&c->ev1));
     // the allocation-free CG's static array on this device (current now) and its code

@@ -30,6 +30,7 @@ constexpr int kRedBlocks = 1024;     // max partials per reduction
 // slot (a slot past its row's length), so kernels need no row lengths;
 // dictionaries therefore hold at most 255 offsets
 constexpr unsigned kPadCode = 255;
+constexpr size_t kReportBytes = 8 << 10;   // pinned reports behind host_res
 constexpr int kHostDot = 255;        // word of host_res that such a dot's result arrives in
 constexpr int kNumXcd = 8;           // MI355X: 8 accelerator complex dies
 // Size of the per-device static array that the allocation-free CG
@@ -58,6 +59,7 @@ struct hfh_ctx {
     // reduction scratch: partials[kRedBlocks * 8] doubles, then result slots
     double *red = nullptr;            // device
     double *host_res = nullptr;       // pinned host mirror for results
+    void *host_reports = nullptr;     // pinned, behind it: rows reported by a search for pairs
     unsigned long long *dot_slots = nullptr;   // partials of dots that the host waits for (in red)
     hfh::Timing timing;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -120,8 +122,6 @@ struct hfh_csr {
     // Matrices of a few distinct (offset, value) pairs (hfh_pattern.hip), on
     // top of an automatically chosen SELL layout of one wave per slice
     bool pt_want = false;          // the layout was chosen automatically
-    bool pt_scanned = false;       // pt_rows is up to date with the structure
-    std::vector<int> pt_rows;      // sample rows of every pattern of offsets (empty: too many)
     int pt_pairs = 0;              // pairs (0: the values do not repeat)
     int pt_omin = 0, pt_omax = 0;  // smallest and largest offset
     int pt_ngroups = 0;            // runs of up to three neighbouring offsets

@@ -17,58 +17,21 @@
 
 #include <algorithm>
 #include <cstring>
-#include <thread>
 
 namespace hfh {
 namespace {
 
-constexpr int kMaxPatterns = 64;   // distinct rows of offsets looked at
 constexpr int kMaxPairs = 32;      // bits of a row's set
-
-// Values of the listed rows, one workgroup per row, at out[g * kMaxPairs].
-template <typename T>
-__global__ void k_pattern_gather(const int *__restrict__ rows, const int *__restrict__ row,
-                                 const T *__restrict__ val, T *__restrict__ out) {
-    const int r = rows[blockIdx.x], j0 = row[r], len = row[r + 1] - j0;
-    const int k = threadIdx.x;
-    if (k < kMaxPairs) out[blockIdx.x * kMaxPairs + k] = k < len ? val[j0 + k] : static_cast<T>(0);
-}
-
-__device__ __forceinline__ bool same_bits(double a, double b) { return __builtin_bit_cast(unsigned long long, a) == __builtin_bit_cast(unsigned long long, b); }
-__device__ __forceinline__ bool same_bits(float a, float b) { return __builtin_bit_cast(unsigned, a) == __builtin_bit_cast(unsigned, b); }
-
-// Every row's set of pairs and, per slice of 64 rows, whether all its rows
-// hold all pairs; *fail when a row has an entry that is no pair.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_pattern_sets(int nrow, int npair, const int *__restrict__ offs,
-                                                         const T *__restrict__ vals, const int *__restrict__ row,
-                                                         const int *__restrict__ col, const T *__restrict__ val,
-                                                         unsigned *__restrict__ set, int *__restrict__ partial,
-                                                         int *fail) {
-    const int r = blockIdx.x * kBlock + threadIdx.x;
-    const unsigned all = npair == 32 ? ~0u : (1u << npair) - 1;
-    unsigned m = 0;
-    bool bad = false;
-    if (r < nrow) {
-        int k = 0;
-        for (int j = row[r]; j < row[r + 1] && !bad; ++j) {
-            const int o = col[j] - r;
-            const T v = val[j];
-            while (k < npair && (offs[k] < o || (offs[k] == o && !same_bits(vals[k], v)))) ++k;
-            if (k < npair && offs[k] == o) m |= 1u << k++;
-            else bad = true;
-        }
-        set[r] = m;
-    }
-    const bool some = __any(r < nrow && m != all);
-    if ((threadIdx.x & 63) == 0 && r < nrow) partial[r >> 6] = some ? 1 : 0;
-    if (bad) *fail = 1;
-}
 
 // Pairs with neighbouring offsets share one load of x.
 struct Group {
     int off;       // offset of the loaded entries: the middle pair of three, else the first
     int bit, n;    // pairs bit .. bit + n - 1, n = 1 .. 3
+};
+
+// Offsets of the pairs, ascending.
+struct Offsets {
+    int v[kMaxPairs];
 };
 
 // The lists as a kernel argument: with compile-time positions all of them
@@ -79,6 +42,127 @@ struct Lists {
     Group grp[kMaxPairs];
     T val[kMaxPairs];
 };
+
+// A row as the host sees it (pinned memory).
+struct RowReport {
+    int len;                       // entries, -1: no report
+    int row;
+    int off[kMaxPairs];
+    unsigned long long val[kMaxPairs];   // the value's bits
+};
+constexpr int kProbes = 8;         // rows spread over the matrix, then the first and the last one
+constexpr int kReports = 16;
+static_assert(kProbes + 2 <= kReports && sizeof(RowReport) * kReports <= kReportBytes, "the context's pinned reports");
+
+__device__ __forceinline__ unsigned long long bits_of(double a) { return __builtin_bit_cast(unsigned long long, a); }
+__device__ __forceinline__ unsigned long long bits_of(float a) { return __builtin_bit_cast(unsigned, a); }
+
+// One lane per entry (the lanes of a wave, of which the first kMaxPairs write).
+template <typename T>
+__device__ __forceinline__ void report_row(RowReport *out, int r, int j0, int len, int lane, const int *__restrict__ col,
+                                           const T *__restrict__ val) {
+    if (lane < min(len, kMaxPairs)) {
+        out->off[lane] = col[j0 + lane] - r;
+        out->val[lane] = bits_of(val[j0 + lane]);
+    }
+    if (lane == 0) {
+        out->row = r;
+        out->len = len;
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(64) void k_pattern_probe(int nrow, const int *__restrict__ row, const int *__restrict__ col,
+                                                      const T *__restrict__ val, RowReport *out, int *count, int rounds) {
+    const int i = blockIdx.x;
+    if (i == 0 && static_cast<int>(threadIdx.x) < rounds) count[threadIdx.x] = 0;
+    const int r = i < kProbes ? static_cast<int>(static_cast<long long>(nrow) * (i + 1) / (kProbes + 1))
+                              : i == kProbes ? 0 : nrow - 1;
+    report_row(out + i, r, row[r], row[r + 1] - row[r], threadIdx.x, col, val);
+}
+
+// Every row's set of pairs and, per slice of 64 rows, whether some row lacks
+// one; a row with an entry that is no pair is reported (one per slice, the
+// first kReports of them), and the sets then mean nothing.
+// One wave per slice, 64 / W rows at a time with W lanes each, so that the
+// entries are read in memory order (a thread per row: 1,851 us on the 127^3
+// Q1 Laplacian in FP64, 177 us this way).  Entry k of a complete row is
+// pair k, so a row's set is mostly the lanes' ballot; the others search.  The
+// offsets also go to memory, for the SpMV.
+template <typename T, int W>
+__global__ __launch_bounds__(kBlock) void k_pattern_sets(int nrow, int nslice, int npair, Lists<T> L, Offsets offs,
+                                                         const int *__restrict__ row, const int *__restrict__ col,
+                                                         const T *__restrict__ val, int *__restrict__ offs_out,
+                                                         unsigned *__restrict__ set, int *__restrict__ partial,
+                                                         int *count, RowReport *out) {
+    __shared__ int s_off[kMaxPairs];
+    __shared__ T s_val[kMaxPairs];
+    __shared__ unsigned s_set[kBlock];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid < kMaxPairs) {
+        s_off[tid] = tid < npair ? offs.v[tid] : 0x7fffffff;
+        s_val[tid] = L.val[tid];
+        if (blockIdx.x == 0) offs_out[tid] = s_off[tid];
+    }
+    s_set[tid] = 0;
+    __syncthreads();
+    const int s = blockIdx.x * (kBlock / 64) + wave;
+    if (s >= nslice) return;
+    unsigned *const sets = s_set + wave * 64;
+    const int r0 = s * 64, rows = min(64, nrow - r0);
+    const int rp = row[r0 + min(lane, rows)], re = row[r0 + rows];   // 65 row pointers of the slice
+    const unsigned all = npair == 32 ? ~0u : (1u << npair) - 1;
+    const int sub = lane / W, k0 = lane % W;
+    int bad = -1;
+#pragma unroll 4
+    for (int q = 0; q < W; ++q) {
+        const int i = q * (64 / W) + sub;          // this lane's row of the slice
+        const int j0 = __shfl(rp, i, 64), up = __shfl(rp, min(i + 1, 63), 64);   // all lanes take part
+        const int j1 = i == 63 ? re : up;
+        const int len = i < rows ? j1 - j0 : 0;
+        unsigned got = 0;
+        bool wrong = len > kMaxPairs;
+        for (int k = k0; __any(k - k0 < min(len, kMaxPairs)); k += W) {
+            bool match = false;
+            if (k < min(len, kMaxPairs)) {
+                const int o = col[j0 + k] - (r0 + i);
+                const unsigned long long v = bits_of(val[j0 + k]);
+                match = s_off[k] == o && bits_of(s_val[k]) == v;
+                if (!match) {
+                    int p = 0;
+                    for (int h = kMaxPairs / 2; h > 0; h >>= 1)
+                        if (s_off[p + h - 1] < o) p += h;
+                    while (p < npair && s_off[p] == o && bits_of(s_val[p]) != v) ++p;
+                    if (p < npair && s_off[p] == o) got |= 1u << p;
+                    else wrong = true;
+                }
+            }
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(match);
+            const unsigned part = static_cast<unsigned>(m >> (sub * W)) & (W == 32 ? ~0u : (1u << (W & 31)) - 1);
+            if (k0 == 0) got |= part << (k - k0);
+        }
+        if (got) atomicOr(&sets[i], got);
+        const unsigned long long w = __builtin_amdgcn_ballot_w64(wrong);
+        if (w && bad < 0) bad = q * (64 / W) + static_cast<int>(__builtin_ctzll(w)) / W;
+    }
+    if (bad >= 0) {
+        int at = 0;
+        if (lane == 0) {   // a look first: thousands of slices' additions would queue up
+            at = __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (at < kReports) at = atomicAdd(count, 1);
+        }
+        at = __builtin_amdgcn_readfirstlane(at);
+        const int j0 = __shfl(rp, bad, 64), up = __shfl(rp, min(bad + 1, 63), 64);
+        const int j1 = bad == 63 ? re : up;
+        if (at < kReports) report_row(out + at, r0 + bad, j0, j1 - j0, lane, col, val);
+    }
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");   // a wave's LDS accesses execute in order
+    const unsigned m = sets[lane];
+    if (lane < rows) set[r0 + lane] = m;
+    const bool some = __any(lane < rows && m != all);
+    if (lane == 0) partial[s] = some ? 1 : 0;
+}
 
 // One wave per slice of 64 rows, lane = row.  The loads of U groups of a
 // slice go out together, each one 64 consecutive entries of x at a scalar
@@ -176,125 +260,131 @@ __global__ __launch_bounds__(kBlock) void k_spmv_pattern(Lists<T> L, int nrow, i
     }
 }
 
+// A value of type T from its bits.
 template <typename T>
-bool same_value(T a, T b) { return std::memcmp(&a, &b, sizeof(T)) == 0; }
-
-bool same_offsets(const hfh_csr *A, int a, int b) {
-    const int *row = A->h_row.data(), *col = A->h_col.data();
-    const int ja = row[a], jb = row[b], len = row[a + 1] - ja;
-    if (row[b + 1] - jb != len) return false;
-    for (int k = 0; k < len; ++k)
-        if (col[ja + k] - a != col[jb + k] - b) return false;
-    return true;
+T value_of(unsigned long long u) {
+    T v;
+    std::memcpy(&v, &u, sizeof(T));   // the low half holds a float (little endian)
+    return v;
 }
 
-template <typename T>
-int fill(hfh_csr *A) {
-    hipStream_t s = A->ctx->stream;
-    const int np = static_cast<int>(A->pt_rows.size()), n = A->nrow, nsl = (n + 63) / 64;
-    // one block: the sets, the slices' flags, the lists, then what only this
-    // function uses (the sample rows, their values, the failure word)
-    const size_t samples = static_cast<size_t>(np) * kMaxPairs * sizeof(T);
-    const size_t at_vals = 0, at_smp = at_vals + kMaxPairs * sizeof(T), at_offs = at_smp + samples, at_rows = at_offs + kMaxPairs * sizeof(int),
-                 at_fail = at_rows + sizeof(int) * np, at_part = at_fail + sizeof(int),
-                 at_set = at_part + sizeof(int) * nsl, bytes = at_set + sizeof(unsigned) * static_cast<size_t>(n);
-    if (!A->pt_block) {
-        const int rc = copy_alloc(A->ctx, &A->pt_block, bytes);
-        if (rc) return rc == HFH_ERR_NOMEM ? HFH_OK : rc;   // the general layout serves
-    }
-    char *blk = static_cast<char *>(A->pt_block);
-    T *d_vals = reinterpret_cast<T *>(blk + at_vals);
-    A->pt_offs = reinterpret_cast<int *>(blk + at_offs);
-    A->pt_partial = reinterpret_cast<int *>(blk + at_part);
-    A->pt_set = reinterpret_cast<unsigned *>(blk + at_set);
-    int *d_rows = reinterpret_cast<int *>(blk + at_rows), *d_fail = reinterpret_cast<int *>(blk + at_fail);
-    T *d_smp = reinterpret_cast<T *>(blk + at_smp);
-    std::vector<T> hv(static_cast<size_t>(np) * kMaxPairs);
-    HFH_HIP(hipMemcpyAsync(d_rows, A->pt_rows.data(), sizeof(int) * np, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_pattern_gather<T>, dim3(np), dim3(64), 0, s, d_rows, A->row, static_cast<const T *>(A->val),
-                       d_smp);
-    HFH_HIP(hipMemcpyAsync(hv.data(), d_smp, samples, hipMemcpyDeviceToHost, s));
-    HFH_HIP(hipStreamSynchronize(s));
-    // the distinct pairs of the sample rows, ascending by offset
-    std::vector<std::pair<int, T>> pairs;
-    for (int i = 0; i < np; ++i) {
-        const int r = A->pt_rows[i], j0 = A->h_row[r], len = A->h_row[r + 1] - j0;
-        for (int k = 0; k < len; ++k) {
-            const int o = A->h_col[j0 + k] - r;
-            const T v = hv[static_cast<size_t>(i) * kMaxPairs + k];
-            bool known = false;
-            for (const auto &q : pairs) known = known || (q.first == o && same_value(q.second, v));
-            if (!known) {
-                if (static_cast<int>(pairs.size()) == kMaxPairs) return HFH_OK;
-                pairs.emplace_back(o, v);
-            }
+// The distinct pairs of a search, ascending by offset.
+struct Found {
+    std::vector<std::pair<int, unsigned long long>> p;
+    // false: more than a set holds
+    bool add(const RowReport &q) {
+        if (q.len > kMaxPairs) return false;
+        for (int k = 0; k < q.len; ++k) {
+            const std::pair<int, unsigned long long> e(q.off[k], q.val[k]);
+            if (std::find(p.begin(), p.end(), e) != p.end()) continue;
+            if (p.size() == static_cast<size_t>(kMaxPairs)) return false;
+            p.push_back(e);
         }
+        return true;
     }
-    if (pairs.empty()) return HFH_OK;
-    std::stable_sort(pairs.begin(), pairs.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
-    const int K = static_cast<int>(pairs.size());
-    Lists<T> L{};
-    std::vector<int> ho(K);
-    for (int k = 0; k < K; ++k) {
-        ho[k] = pairs[k].first;
-        L.val[k] = pairs[k].second;
-    }
-    // runs of up to three neighbouring offsets; an offset with several values
-    // stands alone, as a row adds its pairs in the order of the list
-    int ngroup = 0;
-    auto alone = [&](int k) { return (k > 0 && ho[k - 1] == ho[k]) || (k + 1 < K && ho[k + 1] == ho[k]); };
-    bool tri = true;
-    for (int k = 0; k < K;) {
-        int c = 1;
-        while (c < 3 && k + c < K && !alone(k) && !alone(k + c) && ho[k + c] == ho[k] + c) ++c;
-        L.grp[ngroup++] = Group{c == 3 ? ho[k] + 1 : ho[k], k, c};
-        tri = tri && c == 3;
-        k += c;
-    }
-    int fail = 0;
-    HFH_HIP(hipMemcpyAsync(A->pt_offs, ho.data(), sizeof(int) * K, hipMemcpyHostToDevice, s));
-    HFH_HIP(hipMemcpyAsync(d_vals, L.val, sizeof(T) * K, hipMemcpyHostToDevice, s));
-    HFH_HIP(hipMemcpyAsync(d_fail, &fail, sizeof(int), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_pattern_sets<T>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, n, K, A->pt_offs,
-                       d_vals, A->row, A->col, static_cast<const T *>(A->val), A->pt_set, A->pt_partial, d_fail);
-    HFH_HIP(hipMemcpyAsync(&fail, d_fail, sizeof(int), hipMemcpyDeviceToHost, s));
-    HFH_HIP(hipStreamSynchronize(s));
-    if (fail) return HFH_OK;
-    A->pt_pairs = K;
-    A->pt_ngroups = ngroup;
-    const char *lists = reinterpret_cast<const char *>(&L);
-    A->pt_lists.assign(lists, lists + sizeof(L));
-    A->pt_tri = tri;
-    A->pt_omin = ho[0];
-    A->pt_omax = ho[K - 1];
-    return HFH_OK;
-}
+};
 
 // Rows spread over the matrix: false when three of them with the same offsets
 // hold three different lists of values, so that a matrix of variable
 // coefficients is known without a look at every row.
-template <typename T>
-int probe(const hfh_csr *A, bool *repeat) {
-    constexpr int N = 8;
-    hipStream_t s = A->ctx->stream;
-    T v[N][kMaxPairs];
-    int r[N], len[N];
-    *repeat = false;
-    for (int i = 0; i < N; ++i) {
-        r[i] = static_cast<int>(static_cast<long long>(A->nrow) * (i + 1) / (N + 1));
-        len[i] = A->h_row[r[i] + 1] - A->h_row[r[i]];
-        if (len[i] > kMaxPairs) return HFH_OK;
-        if (len[i] > 0)
-            HFH_HIP(hipMemcpyAsync(v[i], static_cast<const T *>(A->val) + A->h_row[r[i]], sizeof(T) * len[i],
-                                   hipMemcpyDeviceToHost, s));
-    }
-    HFH_HIP(hipStreamSynchronize(s));
-    auto differ = [&](int i, int j) { return same_offsets(A, r[i], r[j]) && std::memcmp(v[i], v[j], sizeof(T) * len[i]) != 0; };
-    for (int i = 0; i < N; ++i)
+bool repeats(const RowReport *q) {
+    auto differ = [&](int i, int j) {
+        return q[i].len == q[j].len && std::memcmp(q[i].off, q[j].off, sizeof(int) * q[i].len) == 0 &&
+               std::memcmp(q[i].val, q[j].val, sizeof(q[i].val[0]) * q[i].len) != 0;
+    };
+    for (int i = 0; i < kProbes; ++i)
         for (int j = 0; j < i; ++j)
             for (int k = 0; k < j; ++k)
-                if (differ(i, j) && differ(j, k) && differ(i, k)) return HFH_OK;
-    *repeat = true;
+                if (differ(i, j) && differ(j, k) && differ(i, k)) return false;
+    return true;
+}
+
+// Rounds of the search: each looks at all rows with the pairs known so far and
+// reports rows that hold others (the classes of boundary rows of a grid).
+constexpr int kRounds = 8;
+
+template <typename T>
+int search(hfh_csr *A) {
+    hfh_ctx *c = A->ctx;
+    hipStream_t s = c->stream;
+    const int n = A->nrow, nsl = (n + 63) / 64;
+    RowReport *rep = static_cast<RowReport *>(c->host_reports);
+    int *count = reinterpret_cast<int *>(c->red);   // rows that hold no known pair, by round
+    const T *val = static_cast<const T *>(A->val);
+    hipLaunchKernelGGL(k_pattern_probe<T>, dim3(kProbes + 2), dim3(64), 0, s, n, A->row, A->col, val, rep, count, kRounds);
+    int rc = launch_check("k_pattern_probe");
+    if (rc) return rc;
+    HFH_HIP(hipStreamSynchronize(s));
+    Found found;
+    for (int i = 0; i < kProbes + 2; ++i)
+        if (!found.add(rep[i])) return HFH_OK;
+    if (!repeats(rep)) return HFH_OK;
+    // one block: the offsets, the slices' flags, the sets
+    const size_t at_part = sizeof(int) * kMaxPairs, at_set = at_part + sizeof(int) * nsl,
+                 bytes = at_set + sizeof(unsigned) * static_cast<size_t>(n);
+    if (!A->pt_block) {
+        rc = copy_alloc(c, &A->pt_block, bytes);
+        if (rc) return rc == HFH_ERR_NOMEM ? HFH_OK : rc;   // the general layout serves
+    }
+    char *blk = static_cast<char *>(A->pt_block);
+    A->pt_offs = reinterpret_cast<int *>(blk);
+    A->pt_partial = reinterpret_cast<int *>(blk + at_part);
+    A->pt_set = reinterpret_cast<unsigned *>(blk + at_set);
+    for (int round = 0; round < kRounds; ++round) {
+        // A row costs its list's pairs whatever it holds: with less than a
+        // quarter of them per row the entries cost less (2^20 rows, FP64; 16
+        // pairs 18.7 us, 4 / 8 entries per row 17.0 / 24.9; 32 pairs 30.0 us,
+        // 4 / 8 / 16 entries 19.2 / 28.5 / 44.7; 8 pairs 11.8 us, 1 / 2
+        // entries 12.3 / 13.9).
+        const int K = static_cast<int>(found.p.size());
+        if (K == 0 || static_cast<long long>(K) * n > 4LL * A->nnz) return HFH_OK;
+        std::sort(found.p.begin(), found.p.end());
+        Lists<T> L{};
+        Offsets O{};
+        for (int k = 0; k < K; ++k) {
+            O.v[k] = found.p[k].first;
+            L.val[k] = value_of<T>(found.p[k].second);
+        }
+        for (int i = 0; i < kReports; ++i) rep[i].len = -1;
+        const dim3 g((nsl + kBlock / 64 - 1) / (kBlock / 64)), bl(kBlock);
+        const long long mean = (A->nnz + static_cast<long long>(n) - 1) / n;
+        if (mean <= 8)
+            hipLaunchKernelGGL((k_pattern_sets<T, 8>), g, bl, 0, s, n, nsl, K, L, O, A->row, A->col, val, A->pt_offs, A->pt_set, A->pt_partial, count + round, rep);
+        else if (mean <= 16)
+            hipLaunchKernelGGL((k_pattern_sets<T, 16>), g, bl, 0, s, n, nsl, K, L, O, A->row, A->col, val, A->pt_offs, A->pt_set, A->pt_partial, count + round, rep);
+        else
+            hipLaunchKernelGGL((k_pattern_sets<T, 32>), g, bl, 0, s, n, nsl, K, L, O, A->row, A->col, val, A->pt_offs, A->pt_set, A->pt_partial, count + round, rep);
+        if ((rc = launch_check("k_pattern_sets"))) return rc;
+        HFH_HIP(hipStreamSynchronize(s));
+        bool complete = true;
+        for (int i = 0; i < kReports; ++i)
+            if (rep[i].len >= 0) {
+                complete = false;
+                if (!found.add(rep[i])) return HFH_OK;
+            }
+        if (!complete) continue;
+        // runs of up to three neighbouring offsets; an offset with several values
+        // stands alone, as a row adds its pairs in the order of the list
+        const int *ho = O.v;
+        int ngroup = 0;
+        auto alone = [&](int k) { return (k > 0 && ho[k - 1] == ho[k]) || (k + 1 < K && ho[k + 1] == ho[k]); };
+        bool tri = true;
+        for (int k = 0; k < K;) {
+            int m = 1;
+            while (m < 3 && k + m < K && !alone(k) && !alone(k + m) && ho[k + m] == ho[k] + m) ++m;
+            L.grp[ngroup++] = Group{m == 3 ? ho[k] + 1 : ho[k], k, m};
+            tri = tri && m == 3;
+            k += m;
+        }
+        A->pt_pairs = K;
+        A->pt_ngroups = ngroup;
+        const char *lists = reinterpret_cast<const char *>(&L);
+        A->pt_lists.assign(lists, lists + sizeof(L));
+        A->pt_tri = tri;
+        A->pt_omin = ho[0];
+        A->pt_omax = ho[K - 1];
+        return HFH_OK;
+    }
     return HFH_OK;
 }
 
@@ -336,81 +426,13 @@ void pattern_free(hfh_csr *A) {
     if (A->pt_block) (void)hipFree(A->pt_block);
     A->pt_block = nullptr;
     A->pt_pairs = 0;
-    A->pt_rows.clear();
-    A->pt_want = A->pt_scanned = false;
-}
-
-// Sample rows: the first and the last row of every pattern of offsets that
-// each host thread's range holds.  None are kept when there are too many
-// patterns, a row is longer than a set can hold or its columns do not ascend
-// (a diagonal-first matrix).
-static void sample(hfh_csr *A) {
-    const int n = A->nrow;
-    const int *row = A->h_row.data(), *col = A->h_col.data();
-    auto same = [&](int a, int b) { return same_offsets(A, a, b); };
-    struct Found {
-        std::vector<int> first, last;
-        bool over = false;
-    };
-    auto add = [&](Found &f, int r, int at) -> int {   // the pattern of row r, or -1 when there are too many
-        if (at >= 0 && same(f.last[at], r)) {
-            f.last[at] = r;
-            return at;
-        }
-        for (size_t i = 0; i < f.first.size(); ++i)
-            if (same(f.first[i], r)) {
-                f.last[i] = r;
-                return static_cast<int>(i);
-            }
-        const int j0 = row[r], j1 = row[r + 1];
-        bool ok = static_cast<int>(f.first.size()) < kMaxPatterns && j1 - j0 <= kMaxPairs;
-        for (int j = j0 + 1; ok && j < j1; ++j) ok = col[j] > col[j - 1];
-        if (!ok) {
-            f.over = true;
-            return -1;
-        }
-        f.first.push_back(r);
-        f.last.push_back(r);
-        return static_cast<int>(f.first.size()) - 1;
-    };
-    const int nt = n < 4096 ? 1 : static_cast<int>(std::min(16u, std::max(1u, std::thread::hardware_concurrency())));
-    std::vector<Found> found(nt);
-    auto scan = [&](int t) {
-        const int lo = static_cast<int>(static_cast<long long>(n) * t / nt);
-        const int hi = static_cast<int>(static_cast<long long>(n) * (t + 1) / nt);
-        int at = -1;
-        for (int r = lo; r < hi && !found[t].over; ++r) at = add(found[t], r, at);
-    };
-    if (nt == 1) {
-        scan(0);
-    } else {
-        std::vector<std::thread> th;
-        for (int t = 0; t < nt; ++t) th.emplace_back(scan, t);
-        for (auto &t : th) t.join();
-    }
-    Found all;
-    for (const Found &f : found) {
-        if (f.over) return;
-        for (int r : f.first)
-            if (add(all, r, -1) < 0) return;
-        for (int r : f.last)
-            if (add(all, r, -1) < 0) return;
-    }
-    A->pt_rows = all.first;
-    for (size_t i = 0; i < all.first.size(); ++i)
-        if (all.last[i] != all.first[i]) A->pt_rows.push_back(all.last[i]);
+    A->pt_want = false;
 }
 
 int pattern_fill(hfh_csr *A) {
     A->pt_pairs = 0;
-    if (!A->pt_want || A->nrow == 0 || A->nnz == 0) return HFH_OK;
-    bool repeat = false;
-    int rc = A->dtype == HFH_F64 ? probe<double>(A, &repeat) : probe<float>(A, &repeat);
-    if (rc || !repeat) return rc;
-    if (!A->pt_scanned) sample(A);
-    A->pt_scanned = true;
-    if (A->pt_rows.empty()) return HFH_OK;
-    return A->dtype == HFH_F64 ? fill<double>(A) : fill<float>(A);
+    if (!A->pt_want || !A->sorted || A->nrow == 0 || A->nnz == 0) return HFH_OK;
+    return A->dtype == HFH_F64 ? search<double>(A) : search<float>(A);
 }
 
 int pattern_spmv(const hfh_csr *A, const void *x, void *y, int mode, const void *w, double *part, const int *done) {

@@ -150,3 +150,28 @@ def test_no_room_for_the_list(pkg, ctx):
         ctx.set_copy_limit(0)
     A.upload_values(val)
     assert A.pattern_pairs() == 27
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_pairs_that_few_rows_hold(pkg, ctx, dtype):
+    """Pairs of single rows far from the probed ones are found in later rounds,
+    at the first and the last row of a slice and in the last, cut slice; a list
+    that grows past a set, and one most rows hold little of, is not taken."""
+    shape = (9, 33, 65)
+    row, col, val = stencil(shape, *box(3))
+    n = len(row) - 1
+    for rows, pairs in (([64 * 50], 28), ([63], 28), ([n - 1], 28), ([64 * 7, 64 * 9 + 63, n - 2], 30),
+                        (list(range(70, 70 + 64 * 5, 64)), 32), (list(range(70, 70 + 64 * 6, 64)), 0)):
+        v = val.copy()
+        for i, r in enumerate(rows):
+            v[row[r] + np.flatnonzero(col[row[r]:row[r + 1]] == r)] = 20.0 + i
+        compare(pkg, ctx, row, col, v, dtype, pairs)
+    # 3 of 12 / 16 pairs per row
+    for k in (12, 16):
+        i, rng = np.arange(4000), np.random.default_rng(k)
+        o = np.sort(np.argsort(rng.random((4000, k)), 1)[:, :3], 1) * 7
+        c = i[:, None] + o
+        m = c < 4000
+        r = np.zeros(4001, np.int32)
+        np.cumsum(m.sum(1), out=r[1:])
+        compare(pkg, ctx, r, c[m].astype(np.int32), np.cos(o[m]), dtype, k if 4 * m.sum() >= k * 4000 else 0)
