@@ -302,7 +302,7 @@ struct ScopedKernelTimer {
 // summed by a finisher kernel (A->nwg partials).
 int spmv_launch(const hfh_csr *A, const void *x, void *y, int mode);
 int spmv_configure(hfh_csr *A, int algo, int p1, int p2);
-int spmv_sell_fill(hfh_csr *A);
+int spmv_sell_fill(hfh_csr *A, bool search = true);
 // After the device columns changed order: diagonal positions, SpMV layout
 // and SELL copy rebuilt from the CSR arrays (host copies already updated).
 int spmv_refresh_structure(hfh_csr *A);
@@ -310,10 +310,12 @@ int spmv_launch_ex(const hfh_csr *A, const void *x, void *y, int mode, const voi
                    const int *done);
 // SpMV by (offset, value) pairs (hfh_pattern.hip): pattern_fill looks at the
 // structure and the values (A->pt_pairs 0 where they do not qualify; waits
-// for the stream), pattern_free forgets them, pattern_spmv launches (as
+// for the stream), pattern_scale follows a scaling of the values (the pairs
+// found stay the pairs, none found stays none: no search), pattern_free forgets them, pattern_spmv launches (as
 // spmv_launch_ex, A->nwg workgroups and partials of the same rows as the SELL
 // kernels).
 int pattern_fill(hfh_csr *A);
+void pattern_scale(hfh_csr *A, double alpha, bool offdiag_only);
 void pattern_free(hfh_csr *A);
 int pattern_spmv(const hfh_csr *A, const void *x, void *y, int mode, const void *w, double *part, const int *done);
 // One Jacobi step xn = update(b - sum_{j != r} a_rj x_j) over the LDS-staged

@@ -63,10 +63,10 @@ __global__ __launch_bounds__(kBlock) void k_diag_range(int r0, int m, const int 
     }
 }
 
-int values_changed(hfh_csr *A) {
+int values_changed(hfh_csr *A, bool search = true) {
     ++A->version;
     A->sell_dirty = true;
-    int rc = spmv_sell_fill(A);
+    int rc = spmv_sell_fill(A, search);
     if (rc) return rc;
     HFH_HIP(hipStreamSynchronize(A->ctx->stream));
     return HFH_OK;
@@ -118,7 +118,9 @@ extern "C" int hfh_csr_scale(hfh_csr *A, double alpha, int offdiag_only) {
             hipLaunchKernelGGL((k_csr_scale<float, false>), dim3(nb), dim3(kBlock), 0, s, A->nrow, A->row, A->col, (float *)A->val, a);
     }
     int rc = launch_check("k_csr_scale");
-    return rc ? rc : values_changed(A);
+    if (rc) return rc;
+    pattern_scale(A, alpha, offdiag_only != 0);
+    return values_changed(A, false);
 }
 
 extern "C" int hfh_csr_zero_rows(hfh_csr *A, const int *rows, int count, double alpha) {

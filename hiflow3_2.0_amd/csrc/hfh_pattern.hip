@@ -388,6 +388,19 @@ int search(hfh_csr *A) {
     return HFH_OK;
 }
 
+template <typename T>
+void scale_lists(hfh_csr *A, T a, bool offdiag_only) {
+    Lists<T> L;
+    std::memcpy(&L, A->pt_lists.data(), sizeof(L));
+    for (int g = 0; g < A->pt_ngroups; ++g) {
+        const Group &q = L.grp[g];
+        const int off = q.n == 3 ? q.off - 1 : q.off;   // of the group's first pair
+        for (int i = 0; i < q.n; ++i)
+            if (!offdiag_only || off + i != 0) L.val[q.bit + i] *= a;   // one rounding, as the entries'
+    }
+    std::memcpy(A->pt_lists.data(), &L, sizeof(L));
+}
+
 template <typename T, bool ADD, bool DOT, int U, bool TRI, bool EXACT>
 void launch_u(const hfh_csr *A, const T *x, T *y, const T *w, double *part, const int *done) {
     Lists<T> L;
@@ -433,6 +446,12 @@ int pattern_fill(hfh_csr *A) {
     A->pt_pairs = 0;
     if (!A->pt_want || !A->sorted || A->nrow == 0 || A->nnz == 0) return HFH_OK;
     return A->dtype == HFH_F64 ? search<double>(A) : search<float>(A);
+}
+
+void pattern_scale(hfh_csr *A, double alpha, bool offdiag_only) {
+    if (A->pt_pairs == 0) return;
+    if (A->dtype == HFH_F64) scale_lists<double>(A, alpha, offdiag_only);
+    else scale_lists<float>(A, static_cast<float>(alpha), offdiag_only);
 }
 
 int pattern_spmv(const hfh_csr *A, const void *x, void *y, int mode, const void *w, double *part, const int *done) {

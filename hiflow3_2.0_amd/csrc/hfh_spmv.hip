@@ -1289,8 +1289,8 @@ static void launch_t(const hfh_csr *A, const void *x, void *y, const void *w, do
 }
 
 // Builds the SELL-64 values and columns from the device CSR (after an
-// upload, a cast or a change of algorithm).
-int spmv_sell_fill(hfh_csr *A) {
+// upload, a cast or a change of algorithm) and searches it for repeated pairs.
+int spmv_sell_fill(hfh_csr *A, bool search) {
     if ((A->spmv_algo != HFH_SPMV_SELL && A->spmv_algo != HFH_SPMV_SELL_DICT && A->spmv_algo != HFH_SPMV_SELL_PAIRS &&
          A->spmv_algo != HFH_SPMV_SELL_LDS) ||
         !A->sell_dirty || A->nrow == 0)
@@ -1307,7 +1307,7 @@ int spmv_sell_fill(hfh_csr *A) {
     int rc = launch_check("k_csr_to_sell");
     if (rc) return rc;
     A->sell_dirty = false;
-    return pattern_fill(A);
+    return search ? pattern_fill(A) : static_cast<int>(HFH_OK);
 }
 
 int spmv_launch_ex(const hfh_csr *A, const void *x, void *y, int mode, const void *w, double *part,

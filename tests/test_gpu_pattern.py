@@ -175,3 +175,41 @@ def test_pairs_that_few_rows_hold(pkg, ctx, dtype):
         r = np.zeros(4001, np.int32)
         np.cumsum(m.sum(1), out=r[1:])
         compare(pkg, ctx, r, c[m].astype(np.int32), np.cos(o[m]), dtype, k if 4 * m.sum() >= k * 4000 else 0)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("what", ["box", "cross", "two diagonals", "band"])
+def test_scaled_values(pkg, ctx, what, dtype):
+    """Scaling keeps the pairs and their rounding: the whole matrix, the entries
+    off the diagonal, a factor that rounds, one that makes pairs equal (0), and
+    new values afterwards."""
+    shape = (12, 13, 70)
+    if what == "band":      # offsets whose runs start, centre and end at 0
+        n = 700
+        c = np.arange(n)[:, None] + np.array([-9, -2, -1, 0, 1, 2, 40])
+        m = (c >= 0) & (c < n)
+        row, col, val = np.concatenate([[0], np.cumsum(m.sum(1))]).astype(np.int32), c[m].astype(np.int32), \
+            np.broadcast_to(np.cos(np.arange(7)), c.shape)[m]
+    elif what == "two diagonals":
+        n = 12 * 13 * 70
+        row, col, val = stencil(shape, *cross(3), diag=5.0 + (np.arange(n) * 2 // n))
+    else:
+        row, col, val = stencil(shape, *(box(3) if what == "box" else cross(3)))
+    n = len(row) - 1
+    A, B = pkg.CsrMatrix(ctx, row, col, val, dtype=dtype), pkg.CsrMatrix(ctx, row, col, val, dtype=dtype)
+    B.set_spmv(pkg.SPMV_SELL_PAIRS, 1)
+    pairs = A.pattern_pairs()
+    assert pairs > 0 and B.pattern_pairs() == 0
+    X, Y, Z = pkg.Vector(ctx, np.random.default_rng(3).standard_normal(n), dtype), pkg.Vector(ctx, n, dtype), pkg.Vector(ctx, n, dtype)
+    for alpha, off in ((-1.0 / 3, False), (0.1, True), (1e-30, False), (1e30, True), (0.0, True), (7.0, False), (0.0, False)):
+        A.scale(alpha, off)
+        B.scale(alpha, off)
+        assert A.pattern_pairs() == pairs
+        A.spmv(X, Y)
+        B.spmv(X, Z)
+        assert np.array_equal(Y.numpy(), Z.numpy())
+    A.upload_values(val.astype(dtype))
+    B.upload_values(val.astype(dtype))
+    A.spmv(X, Y)
+    B.spmv(X, Z)
+    assert A.pattern_pairs() == pairs and np.array_equal(Y.numpy(), Z.numpy()) and Y.nrm2() > 0
