@@ -31,7 +31,8 @@ def banded(n, half, reach, seed=0):
     return row, c[o].astype(np.int32), v[o], rng.standard_normal(n)
 
 
-def check(pkg, oracle, ctx, system, dtype=np.float64, prec=True, x0=None, **kw):
+def check(pkg, oracle, ctx, system, dtype=np.float64, prec=True, x0=None, one=True, **kw):
+    """one: the solve must be one launch (True) or must not be (False)."""
     row, col, val, rhs = system
     val, rhs = val.astype(dtype), rhs.astype(dtype)
     n = len(rhs)
@@ -40,7 +41,9 @@ def check(pkg, oracle, ctx, system, dtype=np.float64, prec=True, x0=None, **kw):
     A = pkg.CsrMatrix(ctx, row, col, val)
     M = pkg.Preconditioner.jacobi(A) if prec else None
     X = pkg.Vector(ctx, np.zeros(n) if x0 is None else x0, dtype)
+    ran = ctx.cg_launches()
     info = pkg.pcg(A, pkg.Vector(ctx, rhs, dtype), X, M, history=True, check=False, **ctl)
+    assert ctx.cg_launches() == (ran[0] + one, ran[1])
     OA = oracle.Csr(row, col, val)
     xo, oi = oracle.cg(OA, rhs, x0=None if x0 is None else x0.astype(dtype), P=oracle.Prec.jacobi(OA) if prec else None,
                        ctrl=(ctl["maxits"], ctl["atol"], ctl["rtol"], ctl["dtol"]))
@@ -61,9 +64,10 @@ def check(pkg, oracle, ctx, system, dtype=np.float64, prec=True, x0=None, **kw):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("n", [1, 2, 63, 511, 512, 513, 1024, 1025, 2048, 2049, 2560, 2561, 131072, 131073, 262145])
+@pytest.mark.parametrize("n", [1, 2, 63, 511, 512, 513, 1024, 1025, 2048, 2049, 2560, 2561, 131072, 131073, 262145,
+                               524288, 524289])
 def test_sizes(pkg, oracle, ctx, n, dtype):
-    check(pkg, oracle, ctx, banded(n, 2, min(40, max(1, n - 1)), seed=n), dtype)
+    check(pkg, oracle, ctx, banded(n, 2, min(40, max(1, n - 1)), seed=n), dtype, one=n <= 4 * 512 * ctx.info()["num_cu"])
 
 
 @pytest.mark.parametrize("half", [0, 1, 2, 3, 4, 5, 7, 8, 13, 14])
@@ -71,14 +75,17 @@ def test_sizes(pkg, oracle, ctx, n, dtype):
 def test_row_lengths(pkg, oracle, ctx, n, half):
     """2 half + 1 entries: 5, 7, 9, 16 and 28 bound the kernels; 29 takes the launches."""
     for prec in (True, False):
-        check(pkg, oracle, ctx, banded(n, half, 300, seed=half), prec=prec)
+        check(pkg, oracle, ctx, banded(n, half, 300, seed=half), prec=prec, one=half <= 13)
 
 
 @pytest.mark.parametrize("reach", [9000, 15000, 39999])
 def test_windows(pkg, oracle, ctx, reach):
-    """Windows near the LDS size, beyond it (launched form), and as long as the matrix."""
-    check(pkg, oracle, ctx, banded(40000, 2, reach, seed=1))
-    check(pkg, oracle, ctx, banded(40000, 2, reach, seed=1), np.float32)
+    """Windows near the LDS size, beyond it (FP64: launched form), and as long as the matrix."""
+    # 512 rows of a workgroup, the reach on both sides and a zero, in 158 KiB
+    fits = [min(512 + 2 * reach, 40000) + 1 <= 158 * 1024 // size for size in (8, 4)]
+    assert fits == [reach == 9000, True]
+    check(pkg, oracle, ctx, banded(40000, 2, reach, seed=1), one=fits[0])
+    check(pkg, oracle, ctx, banded(40000, 2, reach, seed=1), np.float32, one=fits[1])
 
 
 @pytest.mark.parametrize("n", [1500, 5000])

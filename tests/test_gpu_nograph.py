@@ -23,11 +23,14 @@ from conftest import load_pkg
 P = load_pkg()
 ctx = P.Context(0)
 out = {}
-# CG + Jacobi (graph of 16 iterations per chunk)
+# CG + Jacobi (graph of 16 iterations per chunk; the explicit layout rules the
+# one-launch form out, which has neither graphs nor a loop of launches)
 row, col, val, rhs = P.problem(P.Q1_3D, 21)
 A = P.CsrMatrix(ctx, row, col, val)
+A.set_spmv(P.SPMV_SELL_PAIRS, 1)
 X = P.Vector(ctx, len(rhs))
 inf = P.pcg(A, P.Vector(ctx, rhs), X, P.Preconditioner.jacobi(A), maxits=2000, atol=0.0, rtol=1e-8, history=True)
+assert ctx.cg_launches() == (0, 0)
 out["cg_iters"] = inf["iters"]
 out["cg_hist"] = inf["hist"].tolist()
 out["cg_x"] = X.numpy().tolist()

@@ -774,27 +774,41 @@ def true_res(row, col, val, x, b):
 
 @pytest.mark.parametrize("case,prec", [("q1_2d", "jacobi"), ("fv3", "jacobi"), ("fv3", "none"),
                                        ("q1_3d", "jacobi")])
-def test_pcg_matches_oracle(pkg, ctx, oracle, case, prec):
+@pytest.mark.parametrize("form", ["one launch", "launched"])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_pcg_matches_oracle(pkg, ctx, oracle, case, prec, form, dtype):
+    """Both forms of CG: the automatic layout of systems that fit on the chip
+    takes one launch, an explicit layout the launches."""
     if case == "q1_2d":
         row, col, val, rhs = pkg.problem(pkg.Q1_2D, 63)
     elif case == "q1_3d":
         row, col, val, rhs = pkg.problem(pkg.Q1_3D, 23)
     else:
         row, col, val, rhs = fv3(pkg, 20)
+    f64 = dtype == np.float64
+    val, rhs, rtol = val.astype(dtype), rhs.astype(dtype), 1e-8 if f64 else 1e-4
     A = pkg.CsrMatrix(ctx, row, col, val)
+    if form == "launched":
+        A.set_spmv(pkg.SPMV_SELL_PAIRS, 1)
     P = pkg.Preconditioner.jacobi(A) if prec == "jacobi" else None
-    X = pkg.Vector(ctx, len(rhs))
-    info = pkg.pcg(A, pkg.Vector(ctx, rhs), X, P, maxits=3000, atol=0.0, rtol=1e-8, history=True)
+    X = pkg.Vector(ctx, len(rhs), dtype)
+    ran = ctx.cg_launches()[0]
+    info = pkg.pcg(A, pkg.Vector(ctx, rhs, dtype), X, P, maxits=3000, atol=0.0, rtol=rtol, history=True)
+    assert ctx.cg_launches()[0] - ran == (form == "one launch")
     OA = oracle.Csr(row, col, val)
     xo, oi = oracle.cg(OA, rhs, P=oracle.Prec.jacobi(OA) if prec == "jacobi" else None,
-                       ctrl=(3000, 0.0, 1e-8, 1e6))
+                       ctrl=(3000, 0.0, rtol, 1e6))
     assert info["state"] == pkg.SUCCESS_REL and oi["status"] == oracle.SUCCESS_REL
     assert abs(info["iters"] - oi["iters"]) <= 2
-    k = min(20, len(oi["hist"]), len(info["hist"]))
-    assert np.allclose(info["hist"][:k], oi["hist"][:k], rtol=1e-9)
-    x = X.numpy()
-    assert true_res(row, col, val, x, rhs) < 2e-8
-    assert relnorm(x, xo) < 1e-6
+    # In FP32 the first Ritz values converge after about ten steps of these
+    # systems, and from there the roundings of the lost orthogonality make two
+    # histories part (Paige); before, 8 steps of about 100 eps each are 1e-4.
+    k = min(20 if f64 else 8, len(oi["hist"]), len(info["hist"]))
+    assert np.allclose(info["hist"][:k], oi["hist"][:k], rtol=1e-9 if f64 else 1e-4)
+    if f64:
+        x = X.numpy()
+        assert true_res(row, col, val, x, rhs) < 2e-8
+        assert relnorm(x, xo) < 1e-6
 
 
 def test_pcg_large_grid_matches_oracle(pkg, ctx, oracle):
