@@ -967,6 +967,48 @@ def test_gmres_mgs_cooperative_and_multi_launch(pkg, ctx, oracle, where, dtype):
     assert relnorm(X.numpy(), xo) < (1e-10 if f64 else 1e-4)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("where", ["two_per_thread", "four_per_thread", "eight_per_thread", "above_limit"])
+def test_gmres_nearly_dependent_columns(pkg, ctx, where, dtype):
+    """Eigenvalues in three narrow clusters: from the third column on, A v lies
+    in the span of the basis but for about 1e-7 of it, so Gram-Schmidt cancels
+    nearly everything and the basis loses its orthogonality at the end.  The
+    cooperative sweep takes its vectors in pairs (one of an odd number alone),
+    the other one by one; both must keep GMRES backward stable: the residual
+    ends at a few eps times the condition number, and on the way the estimate
+    of the rotations is the true residual."""
+    per = 1024 * ctx.info()["num_cu"]
+    n = {"two_per_thread": per + 77, "four_per_thread": 3 * per + 5, "eight_per_thread": 5 * per + 13,
+         "above_limit": 8 * per + 1000}[where]
+    rng = np.random.default_rng(21)
+    d = rng.choice([1.0, 10.0, 100.0], n) * (1 + 1e-7 * rng.random(n))
+    r = np.repeat(np.arange(n), 3).reshape(n, 3)
+    c = r + np.array([-1, 0, 1])
+    v = np.stack([-1e-6 * rng.random(n), d, 1e-6 * rng.random(n)], axis=1)
+    keep = (c >= 0) & (c < n)
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(keep.sum(axis=1))
+    col, val = c[keep].astype(np.int32), v[keep].astype(dtype)
+    rhs = rng.uniform(-1, 1, n).astype(dtype)
+    A, B = pkg.CsrMatrix(ctx, row, col, val), pkg.Vector(ctx, rhs, dtype)
+    eps, cond = np.finfo(dtype).eps, 100.0
+
+    def solve(maxits):
+        X = pkg.Vector(ctx, n, dtype)
+        info = pkg.gmres(A, B, X, None, m=12, maxits=maxits, atol=0.0, rtol=1e-30, history=True, check=False)
+        return info, true_res(row, col, val.astype(np.float64), X.numpy().astype(np.float64), rhs.astype(np.float64))
+
+    for steps in (1, 2, 3, 4, 11, 12):    # within one cycle
+        info, true = solve(steps)
+        est = info["hist"][min(steps, info["iters"])] / info["hist"][0]
+        print(f"gmres clusters {where} {np.dtype(dtype).name} {steps}: estimate {est:.3e} true {true:.3e}", flush=True)
+        # each of up to 12 steps adds about an eps of ||A|| ||x|| <= cond ||b||
+        bound = 12 * eps * cond
+        assert abs(est - true) <= 1e-3 * true + bound
+        if steps >= 11:
+            assert true <= bound
+
+
 def test_defect_correction_matches_fp64(pkg, ctx, oracle):
     row, col, val, rhs = fv3(pkg, 20, sigma=1.0, seed=5)
     nc, color, sizes, perm = pkg.multicoloring(row, col)

@@ -122,3 +122,28 @@ def test_no_room_for_the_pencils(pkg, oracle, ctx, shape, limit):
     M.apply(pkg.Vector(ctx, rhs), Y)
     M.sweep_status()
     assert same(Y.numpy(), oracle.sgs(oracle.Csr(row, col, val), rhs))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("shape, bound", [((8, 260, 260), 1089), ((70, 300 * 64 - 7, 1), 300)])
+def test_more_pencils_than_workgroups(pkg, oracle, ctx, shape, bound, dtype):
+    """One workgroup per compute unit and several pencils for each: the tickets,
+    the LDS ring cleared between pencils, the counters handed from sweep to
+    sweep and the inboxes emptied for the next apply."""
+    row, col, val, rhs = system(pkg, shape)
+    val, rhs = val.astype(dtype), rhs.astype(dtype)
+    A = pkg.CsrMatrix(ctx, row, col, val)
+    M = pkg.Preconditioner.sgs(A, row, col)
+    assert M.sweep_blocks()[0] == bound > ctx.info()["num_cu"]
+    M.set_sweep(pkg.SWEEP_SYNCFREE, 1)
+    want = oracle.sgs(oracle.Csr(row, col, val), rhs)
+    X, Y = pkg.Vector(ctx, rhs, dtype), pkg.Vector(ctx, len(rhs), dtype)
+    for _ in range(4):
+        Y.zeros()
+        M.apply(X, Y)
+        M.sweep_status()
+        assert same(Y.numpy(), want)
+    # another right-hand side meets nothing of the last one
+    X.scale(-2.0)
+    M.apply(X, Y)
+    assert same(Y.numpy(), -2 * want)
