@@ -391,6 +391,20 @@ static int resident_rows(const hfh_ctx *c, int n, int L) {
     return 0;
 }
 
+// The most far rows of a window.  A workgroup receives their z in rounds of
+// kPre 512, about 0.3 us per 500 of them, which in the end takes longer than
+// the launched step's three launches (FP32, us per step, one launch /
+// launched; FP64 windows end before, at the LDS's size):
+//   100,000 rows of 5   far 20,000 11.5 / 12.2, 25,000 13.3 / 12.1, 39,000 17.6 / 12.1
+//   260,000 rows of 5   far 20,000 13.5 / 14.1, 22,000 14.1 / 13.9, 39,000 19.1 / 13.9
+//   130,000 rows of 15  far 22,000 12.7 / 13.5, 25,000 13.5 / 13.1
+//   500,000 rows of 5   far 25,000 17.4 / 18.2, 28,000 18.2 / 18.5, 36,000 20.8 / 18.8
+//   500,000 rows of 9   far 32,000 20.1 / 22.0, 36,000 21.4 / 21.2
+//   100,000 rows of 27  far 39,000 17.5 / 18.9; 260,000 rows 19.6 / 26.8
+static int resident_far(int E, int L) {
+    return L > 16 ? 65536 : E < 4 ? 21000 : L <= 5 ? 28000 : 34000;
+}
+
 template <typename T, int L, int E>
 static int resident_launch(const hfh_csr *A, ResidentArgs<T> &a, T *keep, bool noalloc, bool &ran) {
     hfh_ctx *c = A->ctx;
@@ -446,6 +460,7 @@ int cg_resident(const hfh_csr *A, const T *invd, const T *b, T *x, T *z0, T *z1,
     if (E == 0) return HFH_OK;
     const long long window = std::min<long long>(static_cast<long long>(kResBlock) * E + A->shape_lo + A->shape_hi, n) + 1;
     if (window * static_cast<long long>(sizeof(T)) > kResidentLds || window >= 65536) return HFH_OK;
+    if (window - 1 - kResBlock * E > resident_far(E, L)) return HFH_OK;
     ResidentArgs<T> a{n, A->shape_lo, A->shape_hi, A->row, A->col, static_cast<const T *>(A->val), b, invd, x, {z0, z1},
                       reinterpret_cast<unsigned long long *>(slots), hist, c->host_res, ctl.atol, ctl.rtol, ctl.dtol,
                       ctl.maxits, c->wait_polls > 0 ? c->wait_polls : kResPolls};

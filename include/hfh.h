@@ -353,7 +353,7 @@ typedef struct {
  * preconditioning), Jacobi or MC-SGS.  With Jacobi or no preconditioner, an
  * automatic SpMV layout, at most 28 entries per row and a system that fits on
  * the chip (up to 524,288 rows of up to 9 entries, 262,144 otherwise; columns
- * within about 10,000 rows in FP64), the whole solve is one cooperative
+ * within about 10,000 rows, in FP32 up to 19,000 where the rows are long or many), the whole solve is one cooperative
  * launch.  Where one of its bounded waits gives up (other work kept part of
  * its workgroups from starting) the solve begins again from the initial guess
  * in the launched form.  Returns HFH_OK on convergence, HFH_ERR_NOT_CONVERGED on maxits/divergence (info is filled either way).

@@ -78,14 +78,32 @@ def test_row_lengths(pkg, oracle, ctx, n, half):
         check(pkg, oracle, ctx, banded(n, half, 300, seed=half), prec=prec, one=half <= 13)
 
 
-@pytest.mark.parametrize("reach", [9000, 15000, 39999])
-def test_windows(pkg, oracle, ctx, reach):
-    """Windows near the LDS size, beyond it (FP64: launched form), and as long as the matrix."""
-    # 512 rows of a workgroup, the reach on both sides and a zero, in 158 KiB
-    fits = [min(512 + 2 * reach, 40000) + 1 <= 158 * 1024 // size for size in (8, 4)]
-    assert fits == [reach == 9000, True]
-    check(pkg, oracle, ctx, banded(40000, 2, reach, seed=1), one=fits[0])
-    check(pkg, oracle, ctx, banded(40000, 2, reach, seed=1), np.float32, one=fits[1])
+def launches(n, half, reach, size):
+    """Does CG on banded(n, half, reach) take one launch?  Its workgroups' rows,
+    the reach on both sides and a zero must fit 158 KiB of LDS, and the far rows
+    must not take longer than the launches."""
+    rows = 512 * next(e for e in (1, 2, 4) if n <= 512 * 256 * e)
+    far = min(rows + 2 * reach, n) - rows
+    length = 2 * half + 1
+    limit = 65536 if length > 16 else 21000 if rows < 2048 else 28000 if length <= 5 else 34000
+    return (rows + far + 1) * size <= 158 * 1024 and far <= limit
+
+
+@pytest.mark.parametrize("n, half, reach, one64, one32", [
+    (40000, 2, 9000, True, True),       # near the LDS size in FP64
+    (20000, 2, 19999, True, True),      # as long as the matrix
+    (40000, 2, 10500, False, True), (40000, 2, 10501, False, False),    # the far rows
+    (40000, 2, 39999, False, False), (140000, 4, 10501, False, False),
+    (270000, 2, 14000, False, True), (270000, 2, 14001, False, False),
+    (270000, 4, 17000, False, True), (270000, 4, 17001, False, False),
+    (40000, 9, 15000, False, True), (40000, 9, 19000, False, True)])
+def test_windows(pkg, oracle, ctx, n, half, reach, one64, one32):
+    """Windows near the LDS size, beyond it (launched form), as long as the
+    matrix, and with more far rows than pay."""
+    if ctx.info()["num_cu"] >= 256:
+        assert (launches(n, half, reach, 8), launches(n, half, reach, 4)) == (one64, one32)
+    check(pkg, oracle, ctx, banded(n, half, reach, seed=1), one=one64)
+    check(pkg, oracle, ctx, banded(n, half, reach, seed=1), np.float32, one=one32)
 
 
 @pytest.mark.parametrize("n", [1500, 5000])
