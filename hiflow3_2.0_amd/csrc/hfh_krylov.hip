@@ -1093,9 +1093,10 @@ __device__ __forceinline__ void coop_step_sums(const double (&v)[kCoopSums], uns
 // Gram-Schmidt coefficients are h_i = s0 and h_{i+1} = (w - h_i v_i).v_{i+1} =
 // s1 - h_i g.  Between two sums the memory idles while the sum is formed,
 // travels and w is updated, so a sum for two vectors halves that: upwind
-// 128^3 GMRES(30) + ILU(0) 94.5 -> 92.2 ms.  The workgroup's 128 registers
-// per thread hold w and two pairs with a few spilled; 512 threads of 16
-// elements each ran the same.
+// 128^3 GMRES(30) + ILU(0) 94.5 -> 92.2 ms.  At E = 8 in FP64 w and
+// two pairs take more than the workgroup's 128 registers per thread: 37 are
+// spilled (132 bytes of scratch a lane, 33 MiB of a column's writes); 512
+// threads of 16 elements each ran the same.
 template <typename T, int E>
 __global__ __launch_bounds__(kCoopBlock) void k_mgs_coop(int n, const T *__restrict__ w, T *const *__restrict__ V,
                                                          int j, unsigned long long *slots, int nstep, int par,

@@ -33,7 +33,7 @@
 //
 // Measured (apply, both sweeps, FP64; blocks -> pencils): upwind 128^3 ILU(0)
 // 480 -> 267 us, SGS 529 -> 284 us; 2D 701 x 509 SGS 896 -> 427 us; 40^3 SGS
-// 136 -> 86 us; 16^3 51 -> 35 us; 64 x 64 90 -> 49 us.  A step took about 150
+// 136 -> 86 us; 16^3 51 -> 39 us; 64 x 64 89 -> 50 us.  A step took about 150
 // ns and a hop to the next pencil about 2 us on top of its skew.  The step is
 // bound by what a lone wave issues: a dependent FP64 operation 6 to 7 cycles, an
 // LDS write and read back 66, a lane shift of a double 31, a branch on lanes'

@@ -1858,9 +1858,11 @@ static int create_trsv(const hfh_csr *A, int kind, int nlev, const int *lp, cons
     int gnx = 0;
     long long gnxy = 0;
     const bool grid = !rc && detect_grid(A, gnx, gnxy);
-    // full 5- / 7-point stencils stream by pencils at every size (16^3 SGS
-    // 51 us by blocks, 35 us by pencils; 128^3 529 and 284 us); the blocks
-    // remain for the wider stencils and incomplete patterns
+    // full 5- / 7-point stencils stream by pencils at every size from
+    // detect_grid's 4,096 rows on (16^3 SGS 51 us by blocks, 39 us by pencils;
+    // 128^3 529 and 284 us) and at every shape whose pencils are not mostly
+    // skew; the blocks remain for those, the wider stencils and incomplete
+    // patterns
     if (grid) rc = pencil_build(P, gnx, gnxy);
     if (!rc && grid && P->pen.np == 0) {
         for (int shear = 0; shear < 2 && !rc && P->blo.nslice == 0; ++shear)

@@ -901,7 +901,6 @@ static void free_lds_copy(hfh_csr *A) {
 
 static int round8(long long g) { return static_cast<int>(g >= kNumXcd ? (g + kNumXcd - 1) / kNumXcd * kNumXcd : std::max(g, 1LL)); }
 
-// Configures the SpMV kernel of A (host row pointer in A->h_row).
 // The shape the resident CG needs: the longest row and how far the columns
 // (ascending) reach below and above their row.
 static void row_shape(hfh_csr *A) {
@@ -920,6 +919,7 @@ static void row_shape(hfh_csr *A) {
     A->shape_hi = hi;
 }
 
+// Configures the SpMV kernel of A (host row pointer in A->h_row).
 int spmv_configure(hfh_csr *A, int algo, int p1, int p2) {
     const int n = A->nrow;
     row_shape(A);
