@@ -31,12 +31,13 @@
 // fixed order.
 //
 // Measured per step (Jacobi, FP64; launched -> resident): 1,517 rows (2D FV,
-// one workgroup) 13.8 -> 2.7 us, 8,000 rows (3D Q1) 22.6 -> 6.6, 65,025 rows
-// (2D Q1) 14.8 -> 5.7, 125,000 rows (3D Q1) 22.8 -> 10.0, 250,047 rows (3D FV)
-// 19.3 -> 11.3, 490,000 rows (2D Q1) 30.4 -> 8.0.  The largest form (3D Q1,
-// two rows of 27 entries per thread) takes 10.8 us at 175,616 rows and 13.0 at
-// 250,047; with its codes unpacked once and 86 registers spilled 12.3 and 16.8.  What remains is the two
-// sums (1.8 us each on 128 workgroups) and the far z.
+// one workgroup) 13.8 -> 2.5 us, 8,000 rows (3D Q1) 22.6 -> 6.6, 65,025 rows
+// (2D Q1) 14.8 -> 4.7 to 5.6 from process to process, 125,000 rows (3D Q1)
+// 22.8 -> 9.3, 250,047 rows (3D FV) 19.3 -> 11.3, 490,000 rows (2D Q1) 30.4 ->
+// 8.0.  The largest form (3D Q1, two rows of 27 entries per thread) takes
+// 10.8 us at 175,616 rows and 13.0 at 250,047; with its codes unpacked once and
+// 86 registers spilled 12.3 and 16.8.  What remains is the two sums (1.8 us each
+// on 128 workgroups) and the far z.
 #include "hfh_internal.h"
 
 #include <algorithm>
@@ -376,7 +377,7 @@ __global__ __launch_bounds__(kBlock) void k_resident_fill(int n, U *z0, U *z1, U
 // Rows per thread for a system of n rows, 0 where it does not fit the
 // registers of all CUs (the launched form then streams it; at the largest
 // fitting sizes it takes 1.5 to 3 times as long).  One workgroup, with no sum
-// across the grid, is kept up to four rows per thread (1,517 rows: 2.7 us a
+// across the grid, is kept up to four rows per thread (1,517 rows: 2.5 us a
 // step; five workgroups on 2,500 rows: 4.3); otherwise as few rows per thread
 // as the CUs allow.
 // The slots fit n elements: 1024 G bytes, and n > 512 (G - 1) rows of at
