@@ -6,10 +6,12 @@
 // run and every device).  A one-workgroup finisher kernel sums the partials.
 #include "hfh_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 
 namespace hfh {
 
@@ -30,10 +32,32 @@ bool graphs_enabled() {
     return on;
 }
 
+// The live contexts, whose kept work space an allocation may need (never
+// destroyed: a context may be closed while the process ends).
+static std::mutex &g_ctx_mutex = *new std::mutex;
+static std::vector<hfh_ctx *> &g_ctxs = *new std::vector<hfh_ctx *>;
+
+// Frees the work space that contexts keep between calls (none that a running
+// solve holds: it has taken it out).
+static bool release_kept() {
+    std::lock_guard<std::mutex> lock(g_ctx_mutex);
+    bool any = false;
+    for (hfh_ctx *c : g_ctxs)
+        if (JacobiSpace *W = c->jacobi.exchange(nullptr)) {
+            jacobi_space_free(W);
+            any = true;
+        }
+    return any;
+}
+
 int dev_alloc(void **p, size_t bytes) {
     *p = nullptr;
     if (bytes == 0) bytes = 256;
     hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && release_kept()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         set_error("hipMalloc(%zu bytes): %s", bytes, hipGetErrorString(e));
@@ -471,6 +495,10 @@ extern "C" int hfh_ctx_create(int device, hfh_ctx **out) {
         delete c;
         return rc;
     }
+    {
+        std::lock_guard<std::mutex> lock(g_ctx_mutex);
+        g_ctxs.push_back(c);
+    }
     *out = c;
     return HFH_OK;
 }
@@ -479,6 +507,10 @@ extern "C" int hfh_ctx_destroy(hfh_ctx *c) {
     if (!c) return HFH_OK;
     HFH_CHECK(c->live == 0, HFH_ERR_INVALID, "hfh_ctx_destroy: %d objects still use the context; destroy them first",
               c->live);
+    {
+        std::lock_guard<std::mutex> lock(g_ctx_mutex);
+        g_ctxs.erase(std::remove(g_ctxs.begin(), g_ctxs.end(), c), g_ctxs.end());
+    }
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->red) (void)hipFree(c->red);

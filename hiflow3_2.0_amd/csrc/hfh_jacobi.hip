@@ -171,7 +171,8 @@ __global__ __launch_bounds__(kBlock) void k_b_minus(int n, T *__restrict__ r, co
 
 // The two work vectors and the events of a solve.  The context keeps those of
 // the last solve; a solve takes them out while it runs, so solves of several
-// threads never share them, and puts them back once its stream has passed.
+// threads never share them, and puts them back once its stream has passed.  An
+// allocation that the device has no memory for frees them (dev_alloc).
 // Vectors above kSpaceKeep are not kept: allocating them costs little beside
 // the steps they take.
 constexpr size_t kSpaceKeep = static_cast<size_t>(64) << 20;

@@ -201,3 +201,38 @@ def test_smoother_step_counts(pkg, ctx, mode, dtype):
             y = new if mode == "JACOBI_SMOOTH_NORMAL" else 0.3 * y + 0.7 * new
         # each step rounds about 6 operations on values near |y|; 5 steps
         assert np.max(np.abs(x.numpy() - y)) <= 60 * np.finfo(dtype).eps * max(1.0, np.max(np.abs(y)))
+
+
+def test_kept_work_space_is_given_back(pkg):
+    """The vectors a context keeps after a smoother call make room for an
+    allocation that the device has no memory for."""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value, t.value
+
+    n = 7 << 20      # 56 MiB each
+    ctxs = [pkg.Context(0), pkg.Context(0)]
+    for c in ctxs:
+        i = np.arange(n + 1, dtype=np.int32)
+        A = pkg.CsrMatrix(c, i, i[:-1], np.full(n, 2.0))
+        B, X = pkg.Vector(c, n), pkg.Vector(c, n)
+        pkg.jacobi(A, B, X, mode=pkg.JACOBI_SMOOTH_DAMPED, w=0.7, inner_iter=2, smooth_iter=1)
+        del A, B, X
+        c.sync()
+    kept, total = free()
+    with pytest.raises(pkg.HfhError) as e:
+        pkg.BatchEngine(ctxs[0], max_systems=1, hbm_budget=4 * total)
+    assert e.value.code == pkg.ERR_NOMEM
+    assert free()[0] - kept >= 2 * 2 * 8 * n
+    # and the next call takes new ones
+    A = pkg.CsrMatrix(ctxs[1], i, i[:-1], np.full(n, 2.0))
+    B, X = pkg.Vector(ctxs[1], np.full(n, 3.0)), pkg.Vector(ctxs[1], n)
+    pkg.jacobi(A, B, X, mode=pkg.JACOBI_SMOOTH_NORMAL, inner_iter=1, smooth_iter=1)
+    assert np.array_equal(X.numpy(), np.full(n, 1.5))
+    del A, B, X
+    for c in ctxs:
+        c.close()
